@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "ibp_batch.h"
+#include "ibp_fetch_wide.h"
 #include "ibp_internal.h"
 
 namespace ibp {
@@ -36,7 +37,7 @@ __global__ void batch_reset_kernel(unsigned long long *head)
 // is built per item (two loads per lane); keeping it across items would hold
 // registers for the whole loop.
 template <int ROWS, int KINDS>
-__device__ __forceinline__ void run_item(const TaskDev &t, int64_t b, int64_t e)
+__device__ __forceinline__ void run_item(const TaskDev &t, int64_t b, int64_t e, [[maybe_unused]] uint32_t *wide_lds)
 {
     const FetchParams &p = t.p;
     const bool i32 = p.index != nullptr && t.index_bytes == 4;
@@ -44,11 +45,11 @@ __device__ __forceinline__ void run_item(const TaskDev &t, int64_t b, int64_t e)
     if constexpr ((KINDS & kTasksLarge) != 0) {
         if (KINDS == kTasksLarge || kind == kTasksLarge) {
             if (t.elem_bytes == 8) {
-                if (i32) fetch_large_range<uint64_t, int32_t>(p, b, e, 1);
-                else fetch_large_range<uint64_t, int64_t>(p, b, e, 1);
+                if (i32) fetch_wide_range<uint64_t, int32_t>(p, b, e, wide_lds);
+                else fetch_wide_range<uint64_t, int64_t>(p, b, e, wide_lds);
             } else {
-                if (i32) fetch_large_range<uint32_t, int32_t>(p, b, e, 1);
-                else fetch_large_range<uint32_t, int64_t>(p, b, e, 1);
+                if (i32) fetch_wide_range<uint32_t, int32_t>(p, b, e, wide_lds);
+                else fetch_wide_range<uint32_t, int64_t>(p, b, e, wide_lds);
             }
             return;
         }
@@ -82,6 +83,8 @@ __global__ __launch_bounds__(256) void batch_kernel(const TaskDev *__restrict__ 
                                                     unsigned long long *head, int claim, int dynamic)
 {
     __shared__ int64_t first_item[kLdsTasks];
+    // the waves' LDS for wide rows, in launches that hold such a task
+    __shared__ uint32_t wide_lds[(KINDS & kTasksLarge) ? 4 : 1][(KINDS & kTasksLarge) ? kWideLdsWords : 1];
     const int lane = lane_id();
     const bool staged = ntasks <= kLdsTasks;
     if (staged)
@@ -127,7 +130,7 @@ __global__ __launch_bounds__(256) void batch_kernel(const TaskDev *__restrict__ 
             const int64_t b = (item - t.item_begin) * t.rows_per_item;
             int64_t e = b + t.rows_per_item;
             if (e > t.p.n) e = t.p.n;
-            run_item<ROWS, KINDS>(t, b, e);
+            run_item<ROWS, KINDS>(t, b, e, wide_lds[(KINDS & kTasksLarge) ? wave_in_block_id() : 0]);
         }
     }
 }
@@ -217,6 +220,7 @@ int64_t fill_tasks(const ibp_fetch_task *tasks, int n, const BatchConfig &cfg, i
         d.p.n = t.n;
         const bool host = t.comp_loc == IBP_LOC_HOST || (t.comp_loc == IBP_LOC_AUTO && pointer_is_host(t.comp));
         d.p.first_words = first_words_for(t.vec_size, t.elem_bytes, t.comp_len, host);
+        d.p.host_rows = host ? 1 : 0;
         d.p.err = (t.index || t.offsets) ? index_error_counter() : nullptr;
         d.p.offsets = t.offsets;
         d.p.stream_bytes = t.stream_bytes;

@@ -11,6 +11,7 @@
 #include <atomic>
 
 #include "ibp_fetch_launch.h"
+#include "ibp_fetch_wide.h"
 
 namespace ibp {
 
@@ -39,6 +40,8 @@ int fetch_launch(const FetchParams &p, int elem_bytes, int index_bytes, int impl
         while (rows > 2 && (p.n + rows - 1) / rows < want) rows /= 2;
     }
 #endif
+    // Wider rows of 4- and 8-byte elements: teams of waves (ibp_fetch_wide.h).
+    const bool wide = p.vec_size > kWave && elem_bytes >= 4 && impl != 2 && impl != 3 && impl != 4;
     int64_t waves_needed = p.vec_size <= kWave ? (p.n + rows - 1) / rows : p.n;
     int64_t grid = nblks > 0 ? nblks : (waves_needed * kWave + block - 1) / block;
     int64_t cap = (int64_t)dev.num_cus * g_blocks_per_cu.load();
@@ -53,12 +56,14 @@ int fetch_launch(const FetchParams &p, int elem_bytes, int index_bytes, int impl
         // 52-61): which codec runs, where the rows live, the launch shape.
         const char *kind = (impl == 2 || impl == 3 || impl == 4) ? "transfer baseline"
                            : p.vec_size <= kWave ? (layout == kLayoutSlots ? "wave per row group" : "wave per row group (layout)")
-                                                 : "wave per row";
+                           : wide ? "team of waves per batch of rows"
+                                  : "wave per row";
         dprintf("[ibp] decompress_fetch: %s, impl %d, %s rows, V=%lld, w=%d, n=%lld, grid %lld x %d, rows in flight %d, "
                 "first read %d words, comp_len %d\n",
                 kind, impl, host_resident ? "host (PCIe)" : "device", (long long)p.vec_size, elem_bytes,
                 (long long)p.n, (long long)grid, block, p.vec_size <= kWave ? rows : 1, p.first_words, comp_len);
     }
+    if (wide) return fetch_wide_launch(p, layout, elem_bytes, index_bytes, nblks, stream);
     switch (elem_bytes) {
     case 1: return fetch_launch_width<uint8_t>(p, layout, index_bytes, impl, comp_len, rows, (int)grid, block, stream);
     case 2: return fetch_launch_width<uint16_t>(p, layout, index_bytes, impl, comp_len, rows, (int)grid, block, stream);
@@ -131,7 +136,7 @@ extern "C" int ibp_decompress_fetch_ex(int elem_bytes, void *out, const void *co
     p.n = n;
     const bool host = comp_loc == IBP_LOC_HOST || (comp_loc == IBP_LOC_AUTO && pointer_is_host(comp));
     p.first_words = first_words_for(vec_size, elem_bytes, comp_len, host);
-    p.pad = 0;
+    p.host_rows = host ? 1 : 0;
     p.err = (index || condensed || clustered) ? index_error_counter() : nullptr;
     int lay = kLayoutSlots;
     if (condensed) {
