@@ -18,8 +18,8 @@ OUT = os.path.join(PKG, "libibp.so")
 EXT_OUT = os.path.join(PKG, "_C" + sysconfig.get_config_var("EXT_SUFFIX"))
 OBJ_DIR = os.path.join(PKG, "_build")
 SOURCES = ["ibp_core.hip", "ibp_fetch.hip", "ibp_fetch_u64.hip", "ibp_fetch_u32.hip", "ibp_fetch_narrow.hip",
-           "ibp_fetch_wide.hip",
-           "ibp_pack.hip", "ibp_preproc.hip", "ibp_kmeans.hip", "ibp_batch.hip", "ibp_serve.hip", "ibp_io.hip"]
+           "ibp_fetch_wide.hip", "ibp_pack.hip", "ibp_pack_wide.hip",
+           "ibp_preproc.hip", "ibp_kmeans.hip", "ibp_batch.hip", "ibp_serve.hip", "ibp_io.hip"]
 EXT_SOURCE = "ibp_torch.cpp"
 ARCH = os.environ.get("IBP_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=" + ARCH,

@@ -21,6 +21,7 @@
 #include "ibp_bits.h"
 #include "ibp_fetch_dev.h"
 #include "ibp_internal.h"
+#include "ibp_pack.h"
 #include "ibp_tile.h"
 #include "ibp_wave.h"
 
@@ -306,26 +307,9 @@ __device__ __forceinline__ T small_extract(const SmallCols<T> &c, T x)
 // Bytes of one wave's slot buffer: V words padded to 16 bytes.
 __host__ __device__ __forceinline__ int64_t slot_buf_bytes(int64_t V, int w) { return (V * w + 15) / 16 * 16; }
 
-struct PackParams {
-    const void *in;
-    void *out;
-    int64_t num_vecs;
-    int64_t V;
-    const void *mask;
-    const void *bitval;
-    const int32_t *clusters; // mask row per source row, or nullptr
-    int64_t num_clusters;
-    const int64_t *offsets;  // condensed output: inclusive end byte offset per output row
-    int64_t stream_bytes;
-    const void *index;
-    int64_t n;
-    uint32_t *bitmask; // may be nullptr with a condensed output
-    void *gbuf;        // per-wave slot buffers when they do not fit LDS
-    unsigned long long *err;
-    int split = 1;     // waves of a block sharing one 32-row group (1: a wave per group)
-};
-
-// Pack kernel.  BUF_LDS: the per-wave slot buffer is in LDS (dynamic shared
+// Pack kernel of what the tile, small-row and wide-row kernels leave: rows over
+// 32 KiB, narrow rows with clusters or too few for the tiles, 1- and 2-byte
+// elements.  BUF_LDS: the per-wave slot buffer is in LDS (dynamic shared
 // memory); otherwise in p.gbuf.  CONDENSED: output row i goes to bytes
 // [offsets[i-1], offsets[i]) of the stream, cut at its size; otherwise to the
 // V-element slot i.
@@ -1406,6 +1390,8 @@ int pack_typed(PackParams p, hipStream_t stream)
 template <typename T>
 int pack_width(const PackParams &p, int index_bytes, hipStream_t s)
 {
+    if (sizeof(T) >= 4 && p.V > kWave && p.V * (int64_t)sizeof(T) <= kPackWideMaxBytes)
+        return pack_wide_launch(p, (int)sizeof(T), index_bytes, s);
     const bool i32 = p.index && index_bytes == 4;
     if (p.offsets)
         return i32 ? pack_typed<T, int32_t, true>(p, s) : pack_typed<T, int64_t, true>(p, s);

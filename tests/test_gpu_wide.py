@@ -104,3 +104,40 @@ def test_wide_clusters_inside_a_batch(ibp, oracle, w, v, k):
                                    torch.device("cuda"), None, None if ix is None else torch.from_numpy(ix).cuda(),
                                    clusters=torch.from_numpy(cl).cuda())
         assert torch.equal(got.cpu(), torch.from_numpy(x if ix is None else x[ix]))
+
+
+# team sizes (1, 2, 4, 8 waves) follow from the chunks and the rows; 32 KiB is the widest row a team packs
+@pytest.mark.parametrize("w,v", [(4, 65), (4, 129), (4, 255), (4, 513), (4, 2049), (4, 8192), (4, 8193),
+                                 (8, 65), (8, 127), (8, 256), (8, 257), (8, 1030), (8, 4096), (8, 4097)])
+@pytest.mark.parametrize("n", [37, 4500])
+def test_wide_pack_matches_oracle(ibp, oracle, w, v, n):
+    if n > 1000 and v > 300:
+        n = 70  # many rows only where they change the team
+    rng = np.random.default_rng(77 * w + v + n)
+    dt = np.dtype("i%d" % w)
+    k = 3
+    mask = np.stack([masks_of(kind, v, w, rng) for kind in ("runs", "mixed", "runs")])
+    bitval = rng.integers(0, 2 ** 63, size=(k, v), dtype=np.uint64).astype(mask.dtype) & mask
+    cl = rng.integers(0, k, size=n).astype(np.int32)
+    by = [rows_for(n, mask[c], bitval[c], rng) for c in range(k)]
+    x = np.stack(by)[cl, np.arange(n)].view(dt)
+    m, b = mask.view(dt), bitval.view(dt)
+    md, bd, cd = torch.from_numpy(m).cuda(), torch.from_numpy(b).cuda(), torch.from_numpy(cl).cuda()
+    for clusters in (cl, None):
+        kw = {} if clusters is None else {"clusters": cd}
+        mm, bb = (m, b) if clusters is not None else (m[1], b[1])
+        mmd, bbd = (md, bd) if clusters is not None else (md[1].contiguous(), bd[1].contiguous())
+        comp, bm = oracle.compress(x, mm, bb, clusters=clusters)
+        t = torch.from_numpy(x).cuda()
+        got = ibp.compress_inplace(t, mmd, bbd, **kw)
+        assert np.array_equal(got.cpu().numpy(), bm.view(np.int32))
+        assert np.array_equal(t.cpu().numpy().view(comp.dtype), comp)
+        stream, off = oracle.compress_condensed(x, mm, bb, clusters=clusters)
+        s, o = ibp.compress_condensed(torch.from_numpy(x).cuda(), mmd, bbd, **kw)
+        assert np.array_equal(o.cpu().numpy(), off) and np.array_equal(s.cpu().numpy().view(stream.dtype), stream)
+    idx = rng.integers(0, n, size=n // 2)
+    want, wbm = oracle.compress(x[idx], m[1], b[1])
+    t = torch.from_numpy(x).cuda()
+    got = ibp.compress_inplace(t, md[1].contiguous(), bd[1].contiguous(), torch.from_numpy(idx).cuda())
+    assert np.array_equal(got.cpu().numpy(), wbm.view(np.int32))
+    assert np.array_equal(t.cpu().numpy()[:n // 2].view(want.dtype), want)
