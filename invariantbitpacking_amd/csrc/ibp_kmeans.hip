@@ -24,6 +24,7 @@
 
 #include "ibp_bits.h"
 #include "ibp_internal.h"
+#include "ibp_kmeans_mfma.h"
 #include "ibp_wave.h"
 
 namespace ibp {
@@ -31,31 +32,19 @@ namespace ibp {
 template <typename T>
 using KW = typename std::conditional<sizeof(T) == 8, uint64_t, uint32_t>::type;
 
-// Centroids of the lane-per-row assignment (K <= kRowsK) are also kept by
-// column: cent_cols[j * kRowsK + c] = centroid c's word j (zero for c >= K).
-constexpr int kRowsK = 16;
-
 template <typename T>
-__global__ void km_gather_kernel(const T *data, int64_t V, const int64_t *rows, int K, T *centroids, T *cent_cols)
+__global__ void km_gather_kernel(const T *data, int64_t V, const int64_t *rows, int K, T *centroids)
 {
     const int64_t total = (int64_t)K * V;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (int64_t)gridDim.x * blockDim.x) {
         const int64_t c = g / V, j = g % V;
         const int64_t r = rows[c];
-        const T v = r >= 0 ? data[r * V + j] : T(0);
-        centroids[g] = v;
-        if (cent_cols) cent_cols[j * kRowsK + c] = v;
-    }
-    // the by-column copy's centroids past K are zero
-    if (cent_cols && K < kRowsK) {
-        const int pad = kRowsK - K;
-        for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < pad * V;
-             g += (int64_t)gridDim.x * blockDim.x)
-            cent_cols[(g / pad) * kRowsK + K + g % pad] = T(0);
+        centroids[g] = r >= 0 ? data[r * V + j] : T(0);
     }
 }
 
-// Nearest centroid by popc(x ^ c); equal distances go to the highest index.
+// Nearest centroid by popc(x ^ c), for more than kMfmaK centroids; equal
+// distances go to the highest index.
 // Blocks of four waves.  SPLIT = 1: a wave per group of kAssignRows rows.
 // SPLIT = 4 (rows of at least 256 elements): the four waves share one group
 // and wave w takes the columns j = lane + 64 (w + 4k), which gives a few
@@ -171,198 +160,6 @@ __global__ __launch_bounds__(kWave * kAssignWaves) void km_assign_kernel(const T
             }
         }
         if (sl == 0 && lane < kAssignRows && i0 + lane < N) cluster[i0 + lane] = best;
-    }
-}
-
-// Assignment with a lane per row, for K <= kRowsK centroids (kRowsK
-// distances are computed; those past K are never chosen).
-// Block (t, g) of a (row tiles) x (column groups) grid takes rows
-// 64 t .. 64 t + 63 and the column group's words.  The block copies
-// 64 x kRowsTileBytes of its rows at a time to LDS (each load instruction
-// reads four 128-byte row pieces; the next tile is loaded into registers
-// while the current one is used), then each of its four waves takes a quarter
-// of the tile's words: lane r reads row r's word from LDS and the sixteen
-// centroid words of that column, consecutive in cent_cols, are the same for
-// the whole wave, so they are scalar loads used as instruction operands.  A
-// word costs an XOR and a popcount-accumulate per 32 bits and centroid; no
-// lane exchange is needed.  The four waves' distances are summed in LDS.
-// With one column group the block picks each row's nearest centroid;
-// otherwise it stores its partial distances to part[g][row][c] for
-// km_argmin_kernel.
-constexpr int kRowsWaves = 4;
-constexpr int kRowsTileBytes = 128; // of each row per tile
-
-// d + popc(v) as one v_bcnt_u32_b32 with d as its addend.
-__device__ __forceinline__ int bcnt_acc(uint32_t v, int d)
-{
-    asm("v_bcnt_u32_b32 %0, %1, %0" : "+v"(d) : "v"(v));
-    return d;
-}
-__device__ __forceinline__ int hamming_acc(uint64_t x, uint64_t c, int d)
-{
-    return bcnt_acc((uint32_t)(x >> 32) ^ (uint32_t)(c >> 32), bcnt_acc((uint32_t)x ^ (uint32_t)c, d));
-}
-__device__ __forceinline__ int hamming_acc(uint32_t x, uint32_t c, int d) { return bcnt_acc(x ^ c, d); }
-
-// The kRowsK centroid words of one column (consecutive in cent_cols), read
-// as 64-byte vectors so that a uniform address becomes s_load_dwordx16.
-typedef uint32_t dword16_t __attribute__((ext_vector_type(16)));
-template <typename W>
-struct CentColumn {
-    static constexpr int kVecs = kRowsK * (int)sizeof(W) / 64;
-    dword16_t v[kVecs];
-    __device__ __forceinline__ explicit CentColumn(const W *col)
-    {
-#pragma unroll
-        for (int i = 0; i < kVecs; ++i) v[i] = reinterpret_cast<const dword16_t *>(col)[i];
-    }
-    __device__ __forceinline__ W operator[](int c) const
-    {
-        if constexpr (sizeof(W) == 8) {
-            const dword16_t &h = v[c / 8];
-            return ((uint64_t)h[2 * (c % 8) + 1] << 32) | h[2 * (c % 8)];
-        } else {
-            return v[0][c];
-        }
-    }
-};
-
-// Nearest of the first K distances; equal distances go to the highest index.
-__device__ __forceinline__ int32_t nearest(const int (&d)[kRowsK], int K)
-{
-    int best = 0, best_d = 0x7fffffff;
-#pragma unroll
-    for (int c = 0; c < kRowsK; ++c)
-        if (c < K && d[c] <= best_d) {
-            best_d = d[c];
-            best = c;
-        }
-    return best;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kWave * kRowsWaves) void km_assign_rows_kernel(const T *__restrict__ data, int64_t N,
-                                                                            int64_t V, const T *__restrict__ cent_cols,
-                                                                            int K, int64_t group_words,
-                                                                            int32_t *__restrict__ cluster,
-                                                                            int32_t *__restrict__ part)
-{
-    using W = KW<T>;
-    constexpr int TW = kRowsTileBytes / (int)sizeof(W); // words of a row per tile
-    constexpr int WPW = TW / kRowsWaves;                // of them per wave
-    constexpr int LOADS = kWave * TW / (kWave * kRowsWaves);
-    __shared__ W tile[kWave][TW + 1];
-    __shared__ int sum[kRowsWaves - 1][kRowsK][kWave];
-    const W *__restrict__ cent = reinterpret_cast<const W *>(cent_cols);
-    const int lane = lane_id();
-    const int wv = wave_in_block_id();
-    const int64_t row0 = (int64_t)blockIdx.x * kWave;
-    const int64_t col0 = (int64_t)blockIdx.y * group_words;
-    const int64_t col1 = col0 + group_words < V ? col0 + group_words : V;
-    // the words this thread copies: tile row q / TW, word q % TW, q = tid + i * block
-    const W *src[LOADS];
-    int dst_row[LOADS], dst_word[LOADS];
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int q = (int)threadIdx.x + i * kWave * kRowsWaves;
-        dst_row[i] = q / TW;
-        dst_word[i] = q % TW;
-        int64_t r = row0 + dst_row[i];
-        if (r >= N) r = N - 1; // rows past N copy the last row; their result is dropped
-        src[i] = reinterpret_cast<const W *>(data) + r * V + dst_word[i];
-    }
-    int d[kRowsK];
-#pragma unroll
-    for (int c = 0; c < kRowsK; ++c) d[c] = 0;
-    W next[LOADS];
-    {
-        const int valid = (int)(col1 - col0 < TW ? col1 - col0 : TW);
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) next[i] = dst_word[i] < valid ? src[i][col0] : W(0);
-    }
-    for (int64_t j0 = col0; j0 < col1; j0 += TW) {
-        const int valid = (int)(col1 - j0 < TW ? col1 - j0 : TW);
-        __syncthreads(); // the previous tile has been read
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) tile[dst_row[i]][dst_word[i]] = next[i];
-        __syncthreads();
-        if (j0 + TW < col1) {
-            const int64_t j1 = j0 + TW;
-            const int valid1 = (int)(col1 - j1 < TW ? col1 - j1 : TW);
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) next[i] = dst_word[i] < valid1 ? src[i][j1] : W(0);
-        }
-        const int w0 = wv * WPW;
-        const int w1 = w0 + WPW < valid ? w0 + WPW : valid;
-        int w = w0;
-        for (; w + 2 <= w1; w += 2) { // two columns' loads in flight together
-            const W x0 = tile[lane][w], x1 = tile[lane][w + 1];
-            const CentColumn<W> c0(cent + (j0 + w) * kRowsK), c1(cent + (j0 + w + 1) * kRowsK);
-#pragma unroll
-            for (int c = 0; c < kRowsK; ++c) d[c] = hamming_acc(x0, c0[c], d[c]);
-#pragma unroll
-            for (int c = 0; c < kRowsK; ++c) d[c] = hamming_acc(x1, c1[c], d[c]);
-        }
-        if (w < w1) {
-            const W x = tile[lane][w];
-            const CentColumn<W> cw(cent + (j0 + w) * kRowsK);
-#pragma unroll
-            for (int c = 0; c < kRowsK; ++c) d[c] = hamming_acc(x, cw[c], d[c]);
-        }
-    }
-    // waves 1..3 hand their distances to wave 0
-    if (wv > 0) {
-#pragma unroll
-        for (int c = 0; c < kRowsK; ++c) sum[wv - 1][c][lane] = d[c];
-    }
-    __syncthreads();
-    if (wv != 0) return;
-#pragma unroll
-    for (int w = 0; w < kRowsWaves - 1; ++w)
-#pragma unroll
-        for (int c = 0; c < kRowsK; ++c) d[c] += sum[w][c][lane];
-    const int64_t r = row0 + lane;
-    if (r >= N) return;
-    if (gridDim.y == 1) {
-        cluster[r] = nearest(d, K);
-    } else {
-        int4 *p = reinterpret_cast<int4 *>(part + ((int64_t)blockIdx.y * gridDim.x * kWave + r) * kRowsK);
-#pragma unroll
-        for (int c = 0; c < kRowsK; c += 4) p[c / 4] = make_int4(d[c], d[c + 1], d[c + 2], d[c + 3]);
-    }
-}
-
-// Sums the column groups' partial distances of each row and picks its
-// nearest centroid (km_assign_rows_kernel with more than one group): thread
-// (row, c) sums distance c over the groups (the 16 threads of a row read 64
-// consecutive bytes per group), then the row's 16 lanes take the minimum of
-// (distance, 15 - c), so equal distances go to the highest index.
-__global__ __launch_bounds__(256) void km_argmin_kernel(int64_t N, int K, int groups, int64_t group_stride,
-                                                        const int32_t *__restrict__ part, int32_t *__restrict__ cluster)
-{
-    const int c = (int)(threadIdx.x % kRowsK);
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < N * kRowsK;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = t / kRowsK;
-        const int32_t *p = part + r * kRowsK + c;
-        const int64_t gs = group_stride * kRowsK;
-        int a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-        int g = 0;
-        for (; g + 4 <= groups; g += 4) {
-            a0 += p[(int64_t)g * gs];
-            a1 += p[(int64_t)(g + 1) * gs];
-            a2 += p[(int64_t)(g + 2) * gs];
-            a3 += p[(int64_t)(g + 3) * gs];
-        }
-        for (; g < groups; ++g) a0 += p[(int64_t)g * gs];
-        const int dist = (a0 + a1) + (a2 + a3);
-        int key = c < K ? (dist << 4) | (kRowsK - 1 - c) : 0x7fffffff;
-#pragma unroll
-        for (int m = 1; m < kRowsK; m <<= 1) {
-            const int o = (int)shfl((uint32_t)key, lane_id() ^ m);
-            key = o < key ? o : key;
-        }
-        if (c == 0) cluster[r] = kRowsK - 1 - (key & (kRowsK - 1));
     }
 }
 
@@ -817,13 +614,14 @@ __global__ void km_majority_kernel(int64_t V, int K, const int32_t *count, const
 // A block per centroid: thread (p, l) takes part p of 32 consecutive parts of
 // chain l, ORs its words, the parts' ORs meet in LDS, and the thread writes
 // its part's prefix ORs starting from the OR of the parts before it.  The
-// majority words come from km_majority_kernel or km_reduce_majority_kernel;
-// with cent_cols the centroid is also stored by column.
+// majority words come from km_majority_kernel, km_reduce_majority_kernel or
+// km_count_mfma_kernel.  pops, if given: the centroids' popcounts.
 template <typename T>
 __global__ __launch_bounds__(1024) void km_construct_kernel(int64_t V, int K, const T *maj, T *centroids,
-                                                            T *cent_cols)
+                                                            int32_t *pops)
 {
     __shared__ T part_or[32][32];
+    __shared__ int32_t pop;
     const int c = blockIdx.x;
     const int l = (int)threadIdx.x % 32, p = (int)threadIdx.x / 32;
     const int64_t chain = (V + 31) / 32;
@@ -837,7 +635,9 @@ __global__ __launch_bounds__(1024) void km_construct_kernel(int64_t V, int K, co
         if (j < V) acc = (T)(acc | src[j]);
     }
     part_or[p][l] = acc;
+    if (threadIdx.x == 0) pop = 0;
     __syncthreads();
+    int mine = 0;
     T run = 0;
     for (int q = 0; q < p; ++q) run = (T)(run | part_or[q][l]);
     for (int64_t i = i0; i < i1; ++i) {
@@ -845,9 +645,14 @@ __global__ __launch_bounds__(1024) void km_construct_kernel(int64_t V, int K, co
         if (j < V) {
             run = (T)(run | src[j]);
             dst[j] = run;
-            if (cent_cols) cent_cols[j * kRowsK + c] = run;
+            mine += popc((KW<T>)run);
         }
     }
+    if (!pops) return;
+    mine = wave_sum(mine);
+    if (lane_id() == 0) atomicAdd(&pop, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) pops[c] = pop;
 }
 
 // create_mask_many at threshold t (ibp_preproc_kmeans.cuh:273-293):
@@ -866,13 +671,9 @@ __global__ void km_masks_kernel(int64_t V, int K, float t, const int32_t *count,
     const int32_t *bs = bits_set + g * B;
     uint64_t val = 0, m = 0;
     for (int k = 0; k < B; ++k) {
-        const float f = (float)bs[k];
-        if (f >= hi) {
-            val |= 1ull << k;
-            m |= 1ull << k;
-        } else if ((double)f <= lo) {
-            m |= 1ull << k;
-        }
+        const int in = km_mask_bit(bs[k], hi, lo);
+        val |= in > 1 ? 1ull << k : 0ull;
+        m |= in ? 1ull << k : 0ull;
     }
     masks[g] = (T)m;
     bitvals[g] = (T)val;
@@ -958,6 +759,115 @@ unsigned blocks_for(int64_t n, int64_t cap = 4096)
     return (unsigned)b;
 }
 
+// p as the GPU sees it: device memory or pinned host memory (nullptr: neither).
+int32_t *device_view(int32_t *p)
+{
+    hipPointerAttribute_t attr;
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (attr.type != hipMemoryTypeDevice && attr.type != hipMemoryTypeHost) return nullptr;
+    return static_cast<int32_t *>(attr.devicePointer);
+}
+
+// Buffers of a k-means workspace.
+enum : int {
+    kKmCent, kKmMaj, kKmCluster, kKmCount, kKmRows, // always
+    kKmHot, kKmPops,                                // up to kMfmaK clusters
+    kKmPlanes,                                      // ... with bit planes
+    kKmPerm, kKmChunks, kKmPart, kKmBits,           // otherwise (bits also with row parts)
+    kKmBuffers
+};
+
+// How a k-means runs and what it needs.
+struct KmPlan {
+    bool mfma, planes, chunked, sort_in_lds;
+    int64_t max_chunks = 0, chunk_rows = 256;
+    int64_t col_tiles, row_blocks, hot_words; // of 16 dwords, of 128 rows; member bits per cluster in words
+    int64_t parts = 1, blocks_per_part = 0;
+    int split = 1;
+    size_t size[kKmBuffers] = {}, at[kKmBuffers], total = 0;
+};
+
+KmPlan plan_kmeans(const DeviceInfo &dev, int w, int64_t N, int64_t V, int K, bool want_planes)
+{
+    KmPlan pl;
+    const int64_t VD = V * w / 4;
+    // Up to 16 clusters: the assignment on the matrix units
+    // (ibp_kmeans_mfma.h).  Waves per 16-row tile: more while the tiles alone
+    // leave the chip short of waves and each wave keeps two steps of 64 bytes;
+    // 16 for rows of 2 MiB and more, whose sums would leave the exact range of
+    // one accumulator.
+    pl.mfma = K <= kMfmaK && N > 0;
+    const int64_t tiles16 = (N + 15) / 16;
+    pl.col_tiles = (VD + 15) / 16;
+    pl.row_blocks = (N + 127) / 128;
+    pl.hot_words = pl.row_blocks * 4;
+    if ((pl.col_tiles >= 32 && tiles16 < (int64_t)dev.num_cus * 8) || VD * 32 >= ((int64_t)1 << 24)) pl.split = 16;
+    else if (pl.col_tiles >= 8 && tiles16 < (int64_t)dev.num_cus * 32) pl.split = 4;
+    // ... and the bit counts, from the rows' bit planes (as large as the rows;
+    // 2 GiB at most).  Two blocks per 16 dword columns see all rows, unless
+    // these blocks leave half the CUs idle with more than four rounds of rows
+    // each: then the rows are cut into parts (two more small kernels per
+    // iteration).
+    const size_t planes_bytes = (size_t)(pl.col_tiles * pl.row_blocks) * 32 * kWave * sizeof(uint32_t);
+    pl.planes = pl.mfma && want_planes && planes_bytes <= (size_t)2 << 30 && pl.row_blocks <= 65535 * 4;
+    if (pl.planes && pl.col_tiles * 4 < dev.num_cus && pl.row_blocks > 4 * kCountWaves) {
+        pl.parts = (int64_t)dev.num_cus / pl.col_tiles;
+        const int64_t most = (pl.row_blocks + kCountWaves - 1) / kCountWaves;
+        if (pl.parts > most) pl.parts = most;
+        if (pl.parts < 1) pl.parts = 1;
+    }
+    pl.blocks_per_part = (pl.row_blocks + pl.parts - 1) / pl.parts;
+    if (pl.row_blocks > 0) pl.parts = (pl.row_blocks + pl.blocks_per_part - 1) / pl.blocks_per_part;
+    // Otherwise the rows are grouped by cluster.  The LDS counting sort (one
+    // block) serves K <= kSortMaxK and up to 2^20 rows, a histogram and scatter
+    // over many blocks more rows; both cut the clusters into chunks of
+    // chunk_rows rows whose partial bit counts (about 256 MiB of them at most)
+    // are summed per cluster.
+    pl.sort_in_lds = K <= kSortMaxK && N <= ((int64_t)1 << 20);
+    const int64_t per_chunk = V * 8 * w * (int64_t)sizeof(int32_t);
+    // (the chunk index is blockIdx.y of the bit count: below 65535)
+    int64_t max_chunks_mem = ((int64_t)256 << 20) / per_chunk;
+    if (max_chunks_mem > 65534) max_chunks_mem = 65534;
+    pl.chunked = !pl.planes && K <= kSortMaxK && max_chunks_mem > K;
+    // 256-row chunks for the one-block sort; beyond it, about eight bit-count
+    // blocks per CU (more, smaller chunks cost more in the per-cluster sums
+    // than they gain)
+    if (pl.chunked && !pl.sort_in_lds) {
+        const int64_t tiles64 = (V + kWave - 1) / kWave;
+        int64_t want = (int64_t)dev.num_cus * 8 / tiles64;
+        if (want < K + 1) want = K + 1;
+        const int64_t rows = (N + want - 1) / want;
+        if (rows > pl.chunk_rows) pl.chunk_rows = rows;
+    }
+    if (pl.chunked && N / pl.chunk_rows + K + 1 > max_chunks_mem)
+        pl.chunk_rows = (N + max_chunks_mem - K - 1) / (max_chunks_mem - K);
+    pl.max_chunks = pl.chunked ? N / pl.chunk_rows + K + 1 : 0;
+    const int64_t n1 = N > 0 ? N : 1;
+    pl.size[kKmCent] = pl.size[kKmMaj] = (size_t)(K * V * w);
+    pl.size[kKmCluster] = sizeof(int32_t) * (size_t)n1;
+    pl.size[kKmCount] = sizeof(int32_t) * 3 * (size_t)K;
+    pl.size[kKmRows] = sizeof(int64_t) * (size_t)K;
+    if (pl.mfma) {
+        pl.size[kKmHot] = sizeof(uint32_t) * (size_t)(kMfmaK * pl.hot_words);
+        pl.size[kKmPops] = sizeof(int32_t) * (size_t)kMfmaK;
+    }
+    if (pl.planes) pl.size[kKmPlanes] = planes_bytes;
+    else pl.size[kKmPerm] = pl.size[kKmCluster];
+    if (!pl.planes || pl.parts > 1) pl.size[kKmBits] = sizeof(int32_t) * (size_t)((int64_t)K * V * 8 * w);
+    if (pl.chunked) {
+        pl.size[kKmChunks] = sizeof(int32_t) * (size_t)(3 * pl.max_chunks + 2 * K + 1);
+        pl.size[kKmPart] = (size_t)(per_chunk * pl.max_chunks);
+    }
+    for (int i = 0; i < kKmBuffers; ++i) { // 256-byte aligned
+        pl.at[i] = pl.total;
+        pl.total += (pl.size[i] + 255) / 256 * 256;
+    }
+    return pl;
+}
+
 template <typename T>
 int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, void *masks, void *bitvals,
                  int32_t *clusters_out, hipStream_t s)
@@ -982,98 +892,47 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
         }
         for (int64_t c = 1; c < m; ++c) init[(size_t)c] = head[(size_t)c];
     }
-    T *cent = nullptr, *maj = nullptr, *cent_cols = nullptr;
-    int32_t *dist = nullptr;
-    int32_t *cluster = nullptr, *count = nullptr, *offset = nullptr, *fill = nullptr, *perm = nullptr, *bits = nullptr;
-    int32_t *chunks = nullptr, *part = nullptr;
-    int64_t *rows = nullptr;
-    const int64_t nbits = (int64_t)K * V * B;
-    // The LDS counting sort (one block) serves K <= kSortMaxK and up to 2^20
-    // rows, a histogram and scatter over many blocks more rows; both cut the
-    // clusters into chunks of chunk_rows rows whose partial bit counts (about
-    // 256 MiB of them at most) are summed per cluster.
-    const bool sort_in_lds = K <= kSortMaxK && N <= ((int64_t)1 << 20);
-    const int64_t per_chunk = V * B * (int64_t)sizeof(int32_t);
-    // (the chunk index is blockIdx.y of the bit count: below 65535)
-    int64_t max_chunks_mem = ((int64_t)256 << 20) / per_chunk;
-    if (max_chunks_mem > 65534) max_chunks_mem = 65534;
-    const bool chunked = K <= kSortMaxK && max_chunks_mem > K;
-    // 256-row chunks for the one-block sort; beyond it, about eight bit-count
-    // blocks per CU (more, smaller chunks cost more in the per-cluster sums
-    // than they gain)
-    int64_t chunk_rows = 256;
-    if (chunked && !sort_in_lds) {
-        const int64_t tiles64 = (V + kWave - 1) / kWave;
-        int64_t want = (int64_t)dev.num_cus * 8 / tiles64;
-        if (want < K + 1) want = K + 1;
-        const int64_t rows = (N + want - 1) / want;
-        if (rows > chunk_rows) chunk_rows = rows;
-    }
-    if (chunked && N / chunk_rows + K + 1 > max_chunks_mem) chunk_rows = (N + max_chunks_mem - K - 1) / (max_chunks_mem - K);
-    const int64_t max_chunks = chunked ? N / chunk_rows + K + 1 : 0;
-    hipError_t e = hipSuccess;
-    // Lane-per-row assignment (K <= kRowsK): row tiles x column groups, about
-    // eight blocks per CU (2 to 8 measured alike on 4096-row blocks), and the
-    // centroids also by column.
-    const bool rows_assign = K <= kRowsK;
-    constexpr int64_t kTileWords = kRowsTileBytes / (int64_t)sizeof(KW<T>);
-    const int64_t row_tiles = (N + kWave - 1) / kWave;
-    int64_t col_groups = 1, group_words = V;
-    if (rows_assign && row_tiles > 0) {
-        const int64_t max_groups = (V + kTileWords - 1) / kTileWords;
-        col_groups = ((int64_t)dev.num_cus * 8 + row_tiles - 1) / row_tiles;
-        if (col_groups > max_groups) col_groups = max_groups;
-        if (col_groups < 1) col_groups = 1;
-        group_words = ((V + col_groups - 1) / col_groups + kTileWords - 1) / kTileWords * kTileWords;
-        col_groups = (V + group_words - 1) / group_words;
-    }
-    // One workspace allocation, cut into 256-byte aligned buffers.
-    const int64_t n1 = N > 0 ? N : 1;
-    const size_t sz_cent = sizeof(T) * (size_t)(K * V);
-    const size_t sz_cols = rows_assign ? sizeof(T) * (size_t)(kRowsK * V) : 0;
-    const size_t sz_dist = col_groups > 1 ? sizeof(int32_t) * (size_t)(col_groups * row_tiles * kWave * kRowsK) : 0;
-    const size_t sz_cluster = sizeof(int32_t) * (size_t)n1;
-    const size_t sz_count = sizeof(int32_t) * 3 * (size_t)K;
-    const size_t sz_bits = sizeof(int32_t) * (size_t)nbits;
-    const size_t sz_rows = sizeof(int64_t) * (size_t)K;
-    const size_t sz_chunks = chunked ? sizeof(int32_t) * (size_t)(3 * max_chunks + 2 * K + 1) : 0;
-    const size_t sz_part = chunked ? (size_t)(per_chunk * max_chunks) : 0;
-    const size_t sizes[] = {sz_cent, sz_cols, sz_dist, sz_cent, sz_cluster, sz_count, sz_cluster, sz_bits, sz_rows,
-                            sz_chunks, sz_part};
-    size_t total = 0;
-    for (size_t b : sizes) total += (b + 255) / 256 * 256;
+
+    KmPlan pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, true);
     unsigned char *ws = nullptr;
-    if ((e = hipMallocAsync((void **)&ws, total, s)) != hipSuccess)
-        return set_error(IBP_ERR_NOMEM, "kmeans workspace allocation failed: %s", hipGetErrorString(e));
-    {
-        size_t at = 0;
-        auto take = [&](size_t b) -> void * {
-            void *p = b ? ws + at : nullptr;
-            at += (b + 255) / 256 * 256;
-            return p;
-        };
-        cent = (T *)take(sz_cent);
-        cent_cols = (T *)take(sz_cols);
-        dist = (int32_t *)take(sz_dist);
-        maj = (T *)take(sz_cent);
-        cluster = (int32_t *)take(sz_cluster);
-        count = (int32_t *)take(sz_count);
-        perm = (int32_t *)take(sz_cluster);
-        bits = (int32_t *)take(sz_bits);
-        rows = (int64_t *)take(sz_rows);
-        chunks = (int32_t *)take(sz_chunks);
-        part = (int32_t *)take(sz_part);
+    hipError_t e = hipMallocAsync((void **)&ws, pl.total, s);
+    if (e != hipSuccess && pl.planes) { // short of memory: the counts without the bit planes
+        (void)hipGetLastError();
+        pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
+        e = hipMallocAsync((void **)&ws, pl.total, s);
     }
+    if (e != hipSuccess) return set_error(IBP_ERR_NOMEM, "kmeans workspace allocation failed: %s", hipGetErrorString(e));
+    auto buf = [&](int i) -> void * { return pl.size[i] ? ws + pl.at[i] : nullptr; };
+    T *const cent = (T *)buf(kKmCent), *const maj = (T *)buf(kKmMaj);
+    uint32_t *const hot = (uint32_t *)buf(kKmHot), *const planes = (uint32_t *)buf(kKmPlanes);
+    int32_t *const cluster = (int32_t *)buf(kKmCluster), *const count = (int32_t *)buf(kKmCount);
+    int32_t *const perm = (int32_t *)buf(kKmPerm), *const bits = (int32_t *)buf(kKmBits);
+    int32_t *const chunks = (int32_t *)buf(kKmChunks), *const part = (int32_t *)buf(kKmPart);
+    int32_t *const pops = (int32_t *)buf(kKmPops);
+    int64_t *const rows = (int64_t *)buf(kKmRows);
+    int32_t *const offset = count + K, *const fill = count + 2 * K;
+    const bool mfma = pl.mfma, use_planes = pl.planes, chunked = pl.chunked, sort_in_lds = pl.sort_in_lds;
+    const int64_t VD = V * (int64_t)sizeof(T) / 4, nbits = (int64_t)K * V * B;
+    const int64_t max_chunks = pl.max_chunks, chunk_rows = pl.chunk_rows;
+    const int64_t col_tiles = pl.col_tiles, row_blocks = pl.row_blocks, hot_words = pl.hot_words;
     auto cleanup = [&]() { (void)hipFreeAsync(ws, s); };
-    offset = count + K;
-    fill = count + 2 * K;
-    if ((e = hipMemcpyAsync(rows, init.data(), sizeof(int64_t) * (size_t)K, hipMemcpyHostToDevice, s)) != hipSuccess) {
-        cleanup();
-        return set_error(IBP_ERR_HIP, "kmeans initialisation failed: %s", hipGetErrorString(e));
+    if (mfma) {
+        KmStart start;
+        for (int c = 0; c < kMfmaK; ++c) start.r[c] = c < K ? init[(size_t)c] : -1;
+        hipLaunchKernelGGL(km_start_kernel, dim3((unsigned)K), dim3(1024), 0, s, (const uint32_t *)data, VD, start,
+                           (uint32_t *)cent, pops);
+        if (use_planes)
+            hipLaunchKernelGGL(km_planes_kernel, dim3((unsigned)col_tiles, (unsigned)((row_blocks + 3) / 4)), dim3(256), 0,
+                               s, (const uint32_t *)data, N, VD, row_blocks, planes);
+    } else {
+        if ((e = hipMemcpyAsync(rows, init.data(), sizeof(int64_t) * (size_t)K, hipMemcpyHostToDevice, s)) != hipSuccess) {
+            cleanup();
+            return set_error(IBP_ERR_HIP, "kmeans initialisation failed: %s", hipGetErrorString(e));
+        }
+        hipLaunchKernelGGL((km_gather_kernel<T>), dim3(blocks_for((int64_t)K * V)), dim3(256), 0, s, data, V, rows, K,
+                           cent);
+        hipLaunchKernelGGL(km_zero_kernel, dim3(blocks_for(N)), dim3(256), 0, s, cluster, N);
     }
-    hipLaunchKernelGGL((km_gather_kernel<T>), dim3(blocks_for((int64_t)K * V)), dim3(256), 0, s, data, V, rows, K, cent,
-                       cent_cols);
-    hipLaunchKernelGGL(km_zero_kernel, dim3(blocks_for(N)), dim3(256), 0, s, cluster, N);
     if ((e = hipGetLastError()) != hipSuccess) {
         cleanup();
         return set_error(IBP_ERR_HIP, "kmeans initialisation failed: %s", hipGetErrorString(e));
@@ -1105,22 +964,44 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
     // chunk sums and majority words in one kernel when every wave's 64
     // counters lie in one cluster
     const bool fused_majority = chunked && (V * B) % kWave == 0;
+    const float sweep_last = sweep_last_threshold();
+    int32_t *const clusters_dev = use_planes ? device_view(clusters_out) : nullptr;
     for (int it = 0; it < 10; ++it) {
-        if (rows_assign) {
-            if (N > 0)
-                hipLaunchKernelGGL((km_assign_rows_kernel<T>), dim3((unsigned)row_tiles, (unsigned)col_groups),
-                                   dim3(kWave * kRowsWaves), 0, s, data, N, V, (const T *)cent_cols, K, group_words,
-                                   cluster, dist);
-            if (col_groups > 1)
-                hipLaunchKernelGGL(km_argmin_kernel, dim3(blocks_for(N * kRowsK)), dim3(256), 0, s, N, K, (int)col_groups,
-                                   row_tiles * kWave, (const int32_t *)dist, cluster);
-        } else if (assign_split)
-            hipLaunchKernelGGL((km_assign_kernel<T, kAssignWaves>), dim3((unsigned)assign_grid),
-                               dim3(kWave * kAssignWaves), 0, s, data, N, V, cent, K, cluster);
-        else
-            hipLaunchKernelGGL((km_assign_kernel<T, 1>), dim3((unsigned)assign_grid), dim3(kWave * kAssignWaves), 0,
-                               s, data, N, V, cent, K, cluster);
-        if (chunked) {
+        if (mfma) {
+            const uint32_t *d = (const uint32_t *)data, *ce = (const uint32_t *)cent;
+            uint16_t *h16 = (uint16_t *)hot;
+            const int64_t hot_tiles = hot_words * 2; // a multiple of 8: whole 128-row blocks
+            // The last assignment goes to the caller's array where the GPU can
+            // write it and nothing here reads it again.
+            int32_t *to = it == 9 && clusters_dev ? clusters_dev : cluster;
+            if (pl.split == 16)
+                hipLaunchKernelGGL((km_assign_mfma_kernel<16>), dim3((unsigned)hot_tiles), dim3(1024), 0, s, d, N, VD, ce, pops,
+                                   K, to, h16, hot_words * 2);
+            else if (pl.split == 4)
+                hipLaunchKernelGGL((km_assign_mfma_kernel<4>), dim3((unsigned)hot_tiles), dim3(256), 0, s, d, N, VD, ce, pops,
+                                   K, to, h16, hot_words * 2);
+            else
+                hipLaunchKernelGGL((km_assign_mfma_kernel<1>), dim3((unsigned)(hot_tiles / 4)), dim3(256), 0, s, d, N,
+                                   VD, ce, pops, K, to, h16, hot_words * 2);
+        } else if (N > 0) {
+            if (assign_split)
+                hipLaunchKernelGGL((km_assign_kernel<T, kAssignWaves>), dim3((unsigned)assign_grid),
+                                   dim3(kWave * kAssignWaves), 0, s, data, N, V, cent, K, cluster);
+            else
+                hipLaunchKernelGGL((km_assign_kernel<T, 1>), dim3((unsigned)assign_grid), dim3(kWave * kAssignWaves), 0,
+                                   s, data, N, V, cent, K, cluster);
+        }
+        if (use_planes) {
+            if (pl.parts > 1) { // bits and count are added to
+                hipLaunchKernelGGL(km_zero_kernel, dim3(blocks_for(nbits)), dim3(256), 0, s, bits, nbits);
+                hipLaunchKernelGGL(km_zero_kernel, dim3(1), dim3(256), 0, s, count, (int64_t)K);
+            }
+            hipLaunchKernelGGL(km_count_mfma_kernel, dim3((unsigned)col_tiles * 2, (unsigned)pl.parts),
+                               dim3(kWave * kCountWaves), 0, s, (const uint32_t *)planes, N, VD, (const uint32_t *)hot,
+                               hot_words, K, pl.blocks_per_part, sweep_last,
+                               it == 9 && pl.parts == 1 ? (uint16_t *)masks : nullptr, (uint16_t *)bitvals, count, bits,
+                               (uint16_t *)maj);
+        } else if (chunked) {
             if (sort_in_lds) {
                 hipLaunchKernelGGL(km_sort_kernel, dim3(1), dim3(1024), 0, s, cluster, N, K, count, offset, perm,
                                    (int)chunk_rows, chunks, chunk_base, chunk_count, nchunks);
@@ -1158,22 +1039,24 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
             hipLaunchKernelGGL((km_bitcount_kernel<T>), dim3(tiles, (unsigned)K, splits), dim3(256), 0, s, data, V,
                                perm, offset, count, bits);
         }
-        if (!fused_majority)
+        if (it == 9) break; // the masks need the counts only
+        if (use_planes ? pl.parts > 1 : !fused_majority)
             hipLaunchKernelGGL((km_majority_kernel<T>), dim3(blocks_for((int64_t)K * V, 1 << 20)), dim3(256), 0, s, V,
                                K, count, bits, maj);
-        hipLaunchKernelGGL((km_construct_kernel<T>), dim3((unsigned)K), dim3(1024), 0, s, V, K, (const T *)maj, cent,
-                           cent_cols);
+        hipLaunchKernelGGL((km_construct_kernel<T>), dim3((unsigned)K), dim3(1024), 0, s, V, K, (const T *)maj, cent, pops);
         e = hipGetLastError();
         if (e != hipSuccess) {
             cleanup();
             return set_error(IBP_ERR_HIP, "kmeans iteration launch failed: %s", hipGetErrorString(e));
         }
     }
-    // Final masks from the last assignment's counts (still in count/bits).
-    hipLaunchKernelGGL((km_masks_kernel<T>), dim3(blocks_for((int64_t)K * V, 1 << 20)), dim3(256), 0, s, V, K,
-                       sweep_last_threshold(), count, bits, (T *)masks, (T *)bitvals);
+    // Final masks from the last assignment's counts (still in count/bits),
+    // unless the counts' blocks have written them.
+    if (!use_planes || pl.parts > 1)
+        hipLaunchKernelGGL((km_masks_kernel<T>), dim3(blocks_for((int64_t)K * V, 1 << 20)), dim3(256), 0, s, V, K,
+                           sweep_last, count, bits, (T *)masks, (T *)bitvals);
     e = hipGetLastError();
-    if (e == hipSuccess && N > 0)
+    if (e == hipSuccess && N > 0 && !clusters_dev)
         e = hipMemcpyAsync(clusters_out, cluster, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s);
     cleanup();
     if (e != hipSuccess) return set_error(IBP_ERR_HIP, "kmeans finish failed: %s", hipGetErrorString(e));
