@@ -75,10 +75,19 @@ int ibp_preprocess(int elem_bytes, const void *data, int64_t num_vecs, int64_t v
  * after srand(seed), computed privately (the process-wide generator is not
  * touched); seed < 0 continues the process-wide rand() state like the
  * reference.  threshold is accepted and ignored, as in the reference.
- * Synchronises the stream before returning. */
+ * Synchronises the stream before returning.  The *_ws form takes device memory
+ * (256-byte aligned) of ibp_preprocess_kmeans_workspace_size() bytes (less runs
+ * too, slower, down to what the call needs without its copy of the rows), or
+ * NULL to let the library allocate (stream-ordered). */
 int ibp_preprocess_kmeans(int elem_bytes, const void *data, int64_t num_vecs, int64_t vec_size,
                           int num_clusters, float threshold, int64_t seed, void *masks,
                           void *bitvals, int32_t *clusters, void *stream);
+size_t ibp_preprocess_kmeans_workspace_size(int elem_bytes, int64_t num_vecs, int64_t vec_size,
+                                            int num_clusters);
+int ibp_preprocess_kmeans_ws(int elem_bytes, const void *data, int64_t num_vecs, int64_t vec_size,
+                             int num_clusters, float threshold, int64_t seed, void *masks,
+                             void *bitvals, int32_t *clusters, void *workspace,
+                             size_t workspace_bytes, void *stream);
 
 /* ---- row layouts -------------------------------------------------------------- */
 

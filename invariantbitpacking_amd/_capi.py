@@ -49,6 +49,8 @@ SIGNATURES = {
     "ibp_preprocess_workspace_size": (_SZ, [_I32, _I64, _F]),
     "ibp_preprocess": (_I32, [_I32, _P, _I64, _I64, _F, _P, _P, _P, _P, _SZ, _P]),
     "ibp_preprocess_kmeans": (_I32, [_I32, _P, _I64, _I64, _I32, _F, _I64, _P, _P, _P, _P]),
+    "ibp_preprocess_kmeans_workspace_size": (_SZ, [_I32, _I64, _I64, _I32]),
+    "ibp_preprocess_kmeans_ws": (_I32, [_I32, _P, _I64, _I64, _I32, _F, _I64, _P, _P, _P, _P, _SZ, _P]),
     "ibp_get_compress_size": (_I32, [_I32, _P, _I64, _I64, _P, _P, _P, _I32, _I64, _P, _P, _P]),
     "ibp_compress": (_I32, [_I32, _P, _P, _I64, _I64, _P, _P, _P, _I32, _I64, _P, _P]),
     "ibp_decompress_fetch": (_I32, [_I32, _P, _P, _I64, _I64, _P, _P, _P, _P, _I32, _I64, _I32, _I32, _I32,

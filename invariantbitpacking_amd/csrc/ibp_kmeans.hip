@@ -870,7 +870,7 @@ KmPlan plan_kmeans(const DeviceInfo &dev, int w, int64_t N, int64_t V, int K, bo
 
 template <typename T>
 int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, void *masks, void *bitvals,
-                 int32_t *clusters_out, hipStream_t s)
+                 int32_t *clusters_out, void *workspace, size_t workspace_bytes, hipStream_t s)
 {
     constexpr int B = 8 * (int)sizeof(T);
     const DeviceInfo &dev = device_info();
@@ -893,15 +893,25 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
         for (int64_t c = 1; c < m; ++c) init[(size_t)c] = head[(size_t)c];
     }
 
+    // The caller's workspace, or an allocation; without the bit planes where
+    // that is too small for them or memory is short.
     KmPlan pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, true);
-    unsigned char *ws = nullptr;
-    hipError_t e = hipMallocAsync((void **)&ws, pl.total, s);
-    if (e != hipSuccess && pl.planes) { // short of memory: the counts without the bit planes
-        (void)hipGetLastError();
-        pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
+    unsigned char *ws = (unsigned char *)workspace;
+    hipError_t e = hipSuccess;
+    if (workspace) {
+        if (workspace_bytes < pl.total) pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
+        if (workspace_bytes < pl.total)
+            return set_error(IBP_ERR_INVALID, "workspace too small (%zu < %zu bytes)", workspace_bytes, pl.total);
+    } else {
         e = hipMallocAsync((void **)&ws, pl.total, s);
+        if (e != hipSuccess && pl.planes) {
+            (void)hipGetLastError();
+            pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
+            e = hipMallocAsync((void **)&ws, pl.total, s);
+        }
+        if (e != hipSuccess)
+            return set_error(IBP_ERR_NOMEM, "kmeans workspace allocation failed: %s", hipGetErrorString(e));
     }
-    if (e != hipSuccess) return set_error(IBP_ERR_NOMEM, "kmeans workspace allocation failed: %s", hipGetErrorString(e));
     auto buf = [&](int i) -> void * { return pl.size[i] ? ws + pl.at[i] : nullptr; };
     T *const cent = (T *)buf(kKmCent), *const maj = (T *)buf(kKmMaj);
     uint32_t *const hot = (uint32_t *)buf(kKmHot), *const planes = (uint32_t *)buf(kKmPlanes);
@@ -915,7 +925,9 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
     const int64_t VD = V * (int64_t)sizeof(T) / 4, nbits = (int64_t)K * V * B;
     const int64_t max_chunks = pl.max_chunks, chunk_rows = pl.chunk_rows;
     const int64_t col_tiles = pl.col_tiles, row_blocks = pl.row_blocks, hot_words = pl.hot_words;
-    auto cleanup = [&]() { (void)hipFreeAsync(ws, s); };
+    auto cleanup = [&]() {
+        if (!workspace) (void)hipFreeAsync(ws, s);
+    };
     if (mfma) {
         KmStart start;
         for (int c = 0; c < kMfmaK; ++c) start.r[c] = c < K ? init[(size_t)c] : -1;
@@ -1070,9 +1082,19 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
 
 using namespace ibp;
 
-extern "C" int ibp_preprocess_kmeans(int elem_bytes, const void *data, int64_t num_vecs, int64_t vec_size,
+extern "C" size_t ibp_preprocess_kmeans_workspace_size(int elem_bytes, int64_t num_vecs, int64_t vec_size,
+                                                       int num_clusters)
+{
+    if ((elem_bytes != 4 && elem_bytes != 8) || vec_size <= 0 || vec_size >= ((int64_t)1 << 24) / elem_bytes ||
+        num_vecs < 0 || num_vecs >= (int64_t)1 << 31 || num_clusters < 1 || num_clusters > 65535)
+        return 0;
+    return plan_kmeans(device_info(), elem_bytes, num_vecs, vec_size, num_clusters, true).total;
+}
+
+extern "C" int ibp_preprocess_kmeans_ws(int elem_bytes, const void *data, int64_t num_vecs, int64_t vec_size,
                                      int num_clusters, float threshold, int64_t seed, void *masks, void *bitvals,
-                                     int32_t *clusters, void *stream)
+                                     int32_t *clusters, void *workspace, size_t workspace_bytes,
+                                        void *stream)
 {
     IBP_TRACE("ibp_preprocess_kmeans");
     (void)threshold; // unused by the reference as well (ibp_preproc_host.cuh:119-284)
@@ -1083,12 +1105,13 @@ extern "C" int ibp_preprocess_kmeans(int elem_bytes, const void *data, int64_t n
     // distances (at most 8 * vec_size * elem_bytes bits) carry a 4-bit
     // centroid tag in an int32
     IBP_CHECK(vec_size * elem_bytes < (int64_t)1 << 24, "rows of 16 MiB or more are not supported");
+    IBP_CHECK((uintptr_t)workspace % 256 == 0, "the workspace must be 256-byte aligned");
     IBP_CHECK(masks && bitvals && ((data && clusters) || num_vecs == 0), "null pointer argument");
     const int st = elem_bytes == 8
                        ? kmeans_typed<uint64_t>(data, num_vecs, vec_size, num_clusters, seed, masks, bitvals, clusters,
-                                                as_stream(stream))
+                                                workspace, workspace_bytes, as_stream(stream))
                        : kmeans_typed<uint32_t>(data, num_vecs, vec_size, num_clusters, seed, masks, bitvals, clusters,
-                                                as_stream(stream));
+                                                workspace, workspace_bytes, as_stream(stream));
     if (st == IBP_OK) dprintf("[ibp] kmeans: K=%d V=%lld N=%lld\n", num_clusters, (long long)vec_size, (long long)num_vecs);
     if (st == IBP_OK && debug_enabled()) {
         // The per-centroid report of the reference's debug build
@@ -1116,6 +1139,14 @@ extern "C" int ibp_preprocess_kmeans(int elem_bytes, const void *data, int64_t n
         dprintf("Finished clustering\n");
     }
     return st;
+}
+
+extern "C" int ibp_preprocess_kmeans(int elem_bytes, const void *data, int64_t num_vecs, int64_t vec_size,
+                                     int num_clusters, float threshold, int64_t seed, void *masks, void *bitvals,
+                                     int32_t *clusters, void *stream)
+{
+    return ibp_preprocess_kmeans_ws(elem_bytes, data, num_vecs, vec_size, num_clusters, threshold, seed, masks, bitvals,
+                                    clusters, nullptr, 0, stream);
 }
 
 extern "C" int ibp_selftest_rand(uint32_t seed, int64_t n)

@@ -1,8 +1,8 @@
 """GPU parity of preprocess_kmeans with up to 16 clusters (products of 0/1
 matrices on the matrix units) at the edges of its tiles: 16-row tiles, 128-row
 blocks, steps of 16 dwords, one, four and sixteen waves per tile, row parts,
-rows whose bit sums pass an accumulator's exact range, tables whose bit planes
-exceed the workspace limit."""
+rows whose bit sums pass an accumulator's exact range, workspaces with and
+without room for the bit planes."""
 import numpy as np
 import pytest
 import torch
@@ -54,3 +54,32 @@ def test_kmeans_rows_of_2_mib(ibp, oracle):
 def test_kmeans_table_in_row_parts(ibp, oracle):
     """A narrow table of many rows: its rows are cut into parts that add up."""
     check(ibp, oracle, groups(700001, 50, 8, 3, seed=2), 2)
+
+
+@pytest.mark.parametrize("n,v,w,k", [(1, 1, 4, 1), (129, 9, 8, 15), (5000, 37, 4, 6), (300, 21, 8, 24), (0, 3, 4, 2)])
+def test_kmeans_workspaces(ibp, oracle, n, v, w, k):
+    """The stated size, the library's own memory, and less down to what the
+    call refuses: every call that runs gives the oracle's result."""
+    from invariantbitpacking_amd import _capi
+    x = groups(n, v, w, max(k, 2), seed=n + v) if n else np.zeros((0, v), "i%d" % w)
+    om, ob, oc = oracle.kmeans(x, k, seed=3)[:3]
+    t = torch.from_numpy(x).cuda()
+    full = _capi.lib().ibp_preprocess_kmeans_workspace_size(w, n, v, k)
+    assert full > 0 and _capi.lib().ibp_preprocess_kmeans_workspace_size(3, n, v, k) == 0
+    ran = []
+    for size in [None, full] + [full * i // 16 for i in range(15, 0, -1)] + [256]:
+        m = torch.full((k, v), 5, dtype=t.dtype, device="cuda")
+        b = torch.full((k, v), 5, dtype=t.dtype, device="cuda")
+        c = torch.full((max(n, 1),), -1, dtype=torch.int32, device="cuda")
+        ws = torch.empty((size or 0) + 1, dtype=torch.uint8, device="cuda")
+        rc = _capi.lib().ibp_preprocess_kmeans_ws(w, t.data_ptr(), n, v, k, -1.0, 3, m.data_ptr(), b.data_ptr(),
+                                                  c.data_ptr(), ws.data_ptr() if size else None, size or 0,
+                                                  torch.cuda.current_stream().cuda_stream)
+        ran.append(rc == 0)
+        if rc:
+            continue
+        assert np.array_equal(c.cpu().numpy()[:n], oc)
+        assert np.array_equal(m.cpu().numpy().view(om.dtype).reshape(om.shape), om)
+        assert np.array_equal(b.cpu().numpy().view(ob.dtype).reshape(ob.shape), ob)
+    assert ran[0] and ran[1] and not ran[-1]
+    assert ran[1:] == sorted(ran[1:], reverse=True)
