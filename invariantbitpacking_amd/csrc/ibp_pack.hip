@@ -22,6 +22,7 @@
 #include "ibp_fetch_dev.h"
 #include "ibp_internal.h"
 #include "ibp_pack.h"
+#include "ibp_slices.h"
 #include "ibp_tile.h"
 #include "ibp_wave.h"
 
@@ -173,6 +174,8 @@ __global__ __launch_bounds__(256) void size_kernel(const T *data, int64_t num_ve
 // those of the elements that are not flagged (lost_step).  Mask and bitval
 // are uniform scalar loads straight from the arguments, a chunk ahead (the
 // last chunk's look-ahead re-reads it), popcounts on the scalar unit.
+// What bounds it: reading the table once; 2,449,029 x 50 doubles: 183 us, 5.35
+// TB/s.
 template <typename T>
 __device__ __forceinline__ void size_score_chunk(const uint4 &v, const T (&m)[16 / sizeof(T)],
                                                  const T (&b)[16 / sizeof(T)], uint32_t &lost)
@@ -254,6 +257,126 @@ __global__ __launch_bounds__(kWave) void size_tile_kernel(const T *__restrict__ 
         // the tile's LDS reads are done before the next copy lands
         __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0)
         __builtin_amdgcn_wave_barrier();
+    }
+    if (total) {
+        // one atomic per wave: the lanes' sums as 24-bit low parts and the
+        // rest (each of 64 fits 32 bits while a lane's sum is below 2^49)
+        const uint32_t lo = (uint32_t)wave_sum((int)(uint32_t)(acc & 0xffffffull));
+        const uint32_t hi = (uint32_t)wave_sum((int)(uint32_t)(acc >> 24));
+        const unsigned long long tot = (unsigned long long)lo + ((unsigned long long)hi << 24);
+        if (lane == 0 && tot) atomicAdd(total, tot);
+    }
+}
+
+// The same for rows of any length of 4- or 8-byte elements from 16 bytes on, in
+// slices that the waves of a block share (ibp_slices.h).
+// What bounds it: reading the table once; 131,588 x 155 doubles: 33 us, 5.0
+// TB/s (a wave per row: 41); 860,675 x 50 floats: 33 us, 5.2 TB/s (93).
+template <typename T, int S, int SPLIT>
+__global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void size_slices_kernel(
+    const T *__restrict__ data, int64_t num_vecs, int64_t V, int nslices, const T *__restrict__ mask,
+    const T *__restrict__ bitval, int64_t *__restrict__ sizes, unsigned long long *total)
+{
+    constexpr int W = (int)sizeof(T);
+    constexpr int EPC = 16 / W;
+    constexpr int WAVES = SPLIT == 1 ? 4 : SPLIT;
+    __shared__ uint4 lds[WAVES][kWave * Slice<S>::STRIDE];
+    __shared__ int32_t flagged;
+    const int lane = lane_id(), wv = wave_in_block_id();
+    if (threadIdx.x == 0) flagged = 0;
+    __syncthreads();
+    int pcs = 0;
+    for (int64_t j = threadIdx.x; j < V; j += blockDim.x) pcs += popc(mask[j]);
+    pcs = wave_sum(pcs);
+    if (lane == 0) atomicAdd(&flagged, pcs);
+    __syncthreads();
+    const uint32_t pcsum = (uint32_t)flagged;
+    uint4 *const mine = lds[wv];
+    const uint4 *const row = mine + lane * Slice<S>::STRIDE;
+    const int C = (int)row_chunks(W, V);
+    const uint32_t row_bytes = (uint32_t)(V * W);
+    const int ntiles = (int)((num_vecs + kWave - 1) / kWave);
+    const int step = SPLIT == 1 ? (int)gridDim.x * WAVES : (int)gridDim.x;
+    const int s0 = SPLIT == 1 ? 0 : wv;
+    const bool any = s0 < nslices;
+    Slice<S> slice;
+    slice.init(row_bytes, lane);
+    struct Unit {
+        T m[EPC], b[EPC];
+    };
+    // The columns of chunk c; those that the row's last chunk shares with the
+    // one before it have no mask there.
+    auto fetch = [&](int c, Unit &u) {
+        const int j0 = c * EPC, first = j0 < (int)V - EPC ? j0 : (int)V - EPC;
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) {
+            u.m[e] = mask[first + e];
+            u.b[e] = bitval[first + e];
+        }
+    };
+    auto need = [&](const Unit &u, const uint4 &v) {
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) asm volatile("" ::"s"(u.m[e]), "s"(u.b[e]));
+        asm volatile("" ::"v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
+    };
+    uint32_t lost;
+    auto score = [&](int c, const Unit &u, const uint4 &v) {
+        const int shared = (c + 1) * EPC - (int)V; // > 0 in a last chunk that is not whole
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) {
+            const T m = e < shared ? T(0) : u.m[e];
+            lost = lost_step<true>(xor_ordered(chunk_elem<T>(v, e), u.b[e]), m, (uint32_t)popc(m), lost);
+        }
+    };
+    int tile = SPLIT == 1 ? (int)blockIdx.x * WAVES + wv : (int)blockIdx.x;
+    if (any && tile < ntiles) slice.load(data, num_vecs, row_bytes, tile, ntiles, s0, nslices, lane);
+    unsigned long long acc = 0;
+    for (; tile < ntiles; tile += step) {
+        lost = 0;
+        for (int s = s0; s < nslices; s += SPLIT) {
+            slice.store(mine, lane);
+            __builtin_amdgcn_wave_barrier();
+            const bool more = s + SPLIT < nslices;
+            if (more || tile + step < ntiles)
+                slice.load(data, num_vecs, row_bytes, more ? tile : tile + step, ntiles, more ? s + SPLIT : s0, nslices,
+                           lane);
+            const int c0 = s * S, nc = C - c0 < S ? C - c0 : S;
+            Unit ua, ub;
+            fetch(c0, ua);
+            uint4 va = row[0], vb;
+            int c = 0;
+            for (; c + 1 < nc; c += 2) {
+                need(ua, va);
+                fetch(c0 + c + 1, ub);
+                vb = row[c + 1];
+                score(c0 + c, ua, va);
+                need(ub, vb);
+                const int next = c + 2 < nc ? c + 2 : c + 1;
+                fetch(c0 + next, ua);
+                va = row[next];
+                score(c0 + c + 1, ub, vb);
+            }
+            if (c < nc) {
+                need(ua, va);
+                score(c0 + c, ua, va);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        const int64_t r = tile * (int64_t)kWave + lane;
+        if constexpr (SPLIT > 1) { // the waves' parts of the rows' losses meet in LDS
+            reinterpret_cast<uint32_t *>(mine)[lane] = lost;
+            __syncthreads();
+            if (wv == 0) {
+#pragma unroll
+                for (int q = 1; q < SPLIT; ++q) lost += reinterpret_cast<const uint32_t *>(lds[q])[lane];
+            }
+            __syncthreads();
+        }
+        if ((SPLIT == 1 || wv == 0) && r < num_vecs) {
+            const int64_t sz = slot_size(V, W, (int64_t)(pcsum - lost));
+            sizes[r] = sz;
+            acc += (unsigned long long)sz;
+        }
     }
     if (total) {
         // one atomic per wave: the lanes' sums as 24-bit low parts and the
@@ -1062,11 +1185,17 @@ __global__ __launch_bounds__(kWave) void pack_tile_condensed_kernel(PackTilePara
 }
 
 // ---- inclusive scan of int64 (the thrust::inclusive_scan of compress_condensed,
-// src/compress.cu:284-285): tile sums, an exclusive scan of the tile sums in
-// one block, then each tile scanned with its carry-in.
+// src/compress.cu:284-285): tile sums, then each tile scanned from the sum of
+// the tiles before it.
+//
+// What bounds it: launches, and the values once in and twice through L2.  Every
+// block adds up the tile sums before its own while these are few; one block
+// scans them first where they are more.  2.45M values: 19 us
+// (strided reads, and the sums scanned in a launch of their own: 41).
 
 constexpr int kScanPer = 16;                  // consecutive values per thread
 constexpr int kScanTile = 256 * kScanPer;     // values per 256-thread block
+constexpr int kScanFew = 2048;                // tile sums that a block adds up by itself
 
 // Inclusive scan over the block's threads (blockDim.x <= 1024) through LDS.
 __device__ __forceinline__ int64_t block_incl_scan(int64_t x, int64_t *lds)
@@ -1084,15 +1213,29 @@ __device__ __forceinline__ int64_t block_incl_scan(int64_t x, int64_t *lds)
     return x;
 }
 
+// Sum over the block of 256 threads, in every thread.
+__device__ __forceinline__ int64_t block_sum(int64_t x, int64_t *lds)
+{
+    const int t = threadIdx.x;
+    lds[t] = x;
+    for (int d = 128; d > 0; d >>= 1) {
+        __syncthreads();
+        if (t < d) lds[t] += lds[t + d];
+    }
+    __syncthreads();
+    return lds[0];
+}
+
 __global__ __launch_bounds__(256) void tile_sum_kernel(const int64_t *v, int64_t n, int64_t *sums)
 {
     __shared__ int64_t lds[256];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPer;
+    const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
     int64_t acc = 0;
+#pragma unroll
     for (int k = 0; k < kScanPer; ++k)
-        if (base + k < n) acc += v[base + k];
-    const int64_t tot = block_incl_scan(acc, lds);
-    if (threadIdx.x == blockDim.x - 1) sums[blockIdx.x] = tot;
+        if (base + k * 256 < n) acc += v[base + k * 256];
+    const int64_t tot = block_sum(acc, lds);
+    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
 __global__ __launch_bounds__(1024) void scan_sums_kernel(int64_t *sums, int64_t ntiles)
@@ -1109,23 +1252,42 @@ __global__ __launch_bounds__(1024) void scan_sums_kernel(int64_t *sums, int64_t 
     }
 }
 
-__global__ __launch_bounds__(256) void tile_scan_kernel(int64_t *v, int64_t n, const int64_t *carry_in)
+// sums: the tiles' sums (scanned = false), or what stands before each tile.
+__global__ __launch_bounds__(256) void tile_scan_kernel(int64_t *v, int64_t n, const int64_t *sums, bool scanned)
 {
-    __shared__ int64_t lds[256];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPer;
+    // the tile in LDS, a gap after every kScanPer values: read and written by
+    // consecutive threads, scanned kScanPer values per thread
+    __shared__ int64_t lds[256], tile[kScanTile + 256];
+    const int t = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * kScanTile;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        const int i = k * 256 + t;
+        tile[i + i / kScanPer] = base + i < n ? v[base + i] : 0;
+    }
+    int64_t before = 0;
+    if (scanned) {
+        before = sums[blockIdx.x];
+    } else {
+        for (int b = t; b < (int)blockIdx.x; b += 256) before += sums[b];
+        before = block_sum(before, lds);
+    }
+    __syncthreads();
     int64_t x[kScanPer];
     int64_t acc = 0;
 #pragma unroll
     for (int k = 0; k < kScanPer; ++k) {
-        x[k] = base + k < n ? v[base + k] : 0;
-        acc += x[k];
+        acc += tile[t * (kScanPer + 1) + k];
+        x[k] = acc;
     }
-    const int64_t incl = block_incl_scan(acc, lds);
-    int64_t run = carry_in[blockIdx.x] + incl - acc;
+    const int64_t run = before + block_incl_scan(acc, lds) - acc;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) tile[t * (kScanPer + 1) + k] = run + x[k];
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < kScanPer; ++k) {
-        run += x[k];
-        if (base + k < n) v[base + k] = run;
+        const int i = k * 256 + t;
+        if (base + i < n) v[base + i] = tile[i + i / kScanPer];
     }
 }
 
@@ -1138,9 +1300,15 @@ int size_typed(const void *data, int64_t num_vecs, int64_t V, const void *mask, 
 {
     const DeviceInfo &dev = device_info();
     if constexpr (sizeof(T) >= 4) {
-        // a whole table with one mask, rows the LDS tiles take: a lane per row
-        if (!index && !clusters && n == num_vecs && n > 0 && tile_rows_ok(V * (int64_t)sizeof(T)) &&
-            ((uintptr_t)data % 16) == 0) {
+        // A whole table with one mask: a lane per row.  Rows of which six
+        // 64-row tiles fit a CU's LDS as they are: tiles of one wave (2,000,000
+        // x 20 doubles: 56 us, slices 63; 448-byte rows, five tiles: 36 and
+        // 24).  Others in slices, but for rows of more than 1 KB that are too
+        // few to give every CU half a tile (4000 x 1100 doubles: slices 14.7
+        // us, a wave per row 9.0; 8000: 16.7 and 17.5).
+        const int64_t row_bytes = V * (int64_t)sizeof(T);
+        const bool whole = !index && !clusters && n == num_vecs && n > 0;
+        if (whole && tile_rows_ok(row_bytes) && row_bytes * kWave * 6 <= 160 * 1024 && ((uintptr_t)data % 16) == 0) {
             const size_t lds = (size_t)kWave * V * sizeof(T);
             int64_t per_cu = (int64_t)(160 * 1024) / (int64_t)lds;
             if (per_cu > 8) per_cu = 8;
@@ -1150,6 +1318,20 @@ int size_typed(const void *data, int64_t num_vecs, int64_t V, const void *mask, 
             hipLaunchKernelGGL((size_tile_kernel<T>), dim3((unsigned)grid), dim3(kWave), lds, stream, (const T *)data,
                                num_vecs, (int)V, (const T *)mask, (const T *)bitval, sizes,
                                (unsigned long long *)total);
+            IBP_LAUNCH_CHECK();
+            return IBP_OK;
+        }
+        if (whole && row_bytes >= 16 && V <= (int64_t)1 << 20 && ((uintptr_t)data % 4) == 0 &&
+            (row_bytes <= 1024 || n >= (int64_t)dev.num_cus * 32)) {
+            const int64_t C = row_chunks((int)sizeof(T), V), ntiles = (n + kWave - 1) / kWave;
+            with_slices(C, ntiles, dev.num_cus, [&](auto s_tag, auto split_tag) {
+                constexpr int S = decltype(s_tag)::value, SPLIT = decltype(split_tag)::value;
+                constexpr int WAVES = SPLIT == 1 ? 4 : SPLIT;
+                const int64_t blocks = SPLIT == 1 ? (ntiles + 3) / 4 : ntiles, most = (int64_t)dev.num_cus * (SPLIT == 16 ? 1 : S == 8 ? 16 / WAVES : 20 / WAVES);
+                hipLaunchKernelGGL((size_slices_kernel<T, S, SPLIT>), dim3((unsigned)(blocks < most ? blocks : most)),
+                                   dim3(kWave * WAVES), 0, stream, (const T *)data, num_vecs, V, (int)((C + S - 1) / S),
+                                   (const T *)mask, (const T *)bitval, sizes, (unsigned long long *)total);
+            });
             IBP_LAUNCH_CHECK();
             return IBP_OK;
         }
@@ -1201,8 +1383,10 @@ int scan_inclusive(int64_t *v, int64_t n, hipStream_t stream, int64_t *tile_sums
     int64_t *sums = tile_sums;
     if (!sums) IBP_HIP(hipMallocAsync((void **)&sums, (size_t)ntiles * sizeof(int64_t), stream));
     hipLaunchKernelGGL(tile_sum_kernel, dim3((unsigned)ntiles), dim3(256), 0, stream, (const int64_t *)v, n, sums);
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, stream, sums, ntiles);
-    hipLaunchKernelGGL(tile_scan_kernel, dim3((unsigned)ntiles), dim3(256), 0, stream, v, n, (const int64_t *)sums);
+    const bool scanned = ntiles > kScanFew;
+    if (scanned) hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, stream, sums, ntiles);
+    hipLaunchKernelGGL(tile_scan_kernel, dim3((unsigned)ntiles), dim3(256), 0, stream, v, n, (const int64_t *)sums,
+                       scanned);
     hipError_t e = hipGetLastError();
     if (!tile_sums) IBP_HIP(hipFreeAsync(sums, stream));
     if (e != hipSuccess) return set_error(IBP_ERR_HIP, "scan kernel launch failed: %s", hipGetErrorString(e));

@@ -11,11 +11,11 @@
 //    device, so the call is asynchronous and never copies to the host.
 #include <stddef.h>
 
-#include <type_traits>
 #include <vector>
 
 #include "ibp_bits.h"
 #include "ibp_internal.h"
+#include "ibp_slices.h"
 #include "ibp_tile.h"
 #include "ibp_wave.h"
 
@@ -118,22 +118,18 @@ struct ScoreRec {
     static constexpr int MASK = (int)sizeof(T) / 4; // dwords of a mask
     static constexpr int COL = (MASK + 1) * NT + MASK;
     static constexpr int STRIDE = (COL * EPU + 3) / 4 * 4;
-    // Where column element e of chunk c stands.
+    // Where column element e of chunk c stands (the row's last chunk ends
+    // with it; columns that it shares with the one before are zero there).
     static __device__ __forceinline__ int64_t at(int64_t c, int e)
     {
         return (c * 2 + e / EPU) * STRIDE + (e % EPU) * COL;
     }
 };
-// Chunks of a row: whole 16 bytes from its start on, and a last one that ends
-// with the row; the columns that it shares with the chunk before it have zero
-// masks in it.
-__host__ __device__ constexpr int64_t score_chunks(int w, int64_t V) { return (V * w + 15) / 16; }
-
 template <typename T, int NT>
 __device__ __forceinline__ void store_rec(uint32_t *recs, int64_t V, int64_t j, const T (&m)[kMaxThresholds], T b)
 {
     using R = ScoreRec<T, NT>;
-    const int64_t C = score_chunks((int)sizeof(T), V);
+    const int64_t C = row_chunks((int)sizeof(T), V);
     auto put = [&](int64_t c, int e, bool zero) {
         uint32_t *r = recs + R::at(c, e);
 #pragma unroll
@@ -343,14 +339,12 @@ __global__ void clear_kernel(Sums *sums) { clear_sums(sums); }
 // columns that are NOT flagged, so S_t = (sum of popcounts) - lost_t needs no
 // cross-lane reduction.
 //
-// Work: 64 rows (a tile) per wave, in slices of S chunks (16 bytes).  A slice's loads are 64 chunks of consecutive rows each; they go to
-// registers while the slice before is scored, then to the wave's own LDS,
-// where lane r reads row r back chunk by chunk (an odd stride of chunks: no
-// bank conflicts).  The columns' constants are uniform, two units per chunk by
-// scalar loads, each issued before the unit in front of it is scored.  SPLIT
-// waves share a tile's slices and meet in LDS.  NT = thresholds of the records; only the first ones, up
-// to the last that flags any bit, are scored (of the sweep over float data,
-// 1.0 and often 0.95 flag nothing).  The tiles are taken from the last one
+// Work: tiles of 64 rows in slices (ibp_slices.h).  The columns' constants are
+// uniform, two units per chunk by scalar loads, each issued before the unit in
+// front of it is scored.  The SPLIT waves of a tile
+// meet in LDS.  NT = thresholds of the records; only the first ones, up to the
+// last that flags any bit, are scored (of the sweep over float data, 1.0 and
+// often 0.95 flag nothing).  The tiles are taken from the last one
 // back: the counts have just read the table's end, so the last-level cache
 // holds it.  The block that finishes last picks the threshold and writes the
 // mask.
@@ -363,8 +357,6 @@ __global__ void clear_kernel(Sums *sums) { clear_sums(sums); }
 // whole call, 614 -> 38 us.  Slices of one wave per tile, whatever the row: 240
 // us; a row's slices follow each other too late to find its lines in L2, so
 // the waves that share a tile load its whole rows together.
-typedef uint32_t score_chunk_t __attribute__((ext_vector_type(4), aligned(4)));
-
 template <typename T, int NT, int S, int SPLIT>
 __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_kernel(
     const T *__restrict__ data, int64_t num_vecs, int64_t V, int nslices, const uint32_t *__restrict__ recs,
@@ -373,8 +365,7 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
 {
     using R = ScoreRec<T, NT>;
     constexpr int WAVES = SPLIT == 1 ? 4 : SPLIT;
-    constexpr int STRIDE = S | 1; // chunks of a row in LDS
-    static_assert(S % 2 || kWave % S == 0, "");
+    constexpr int STRIDE = Slice<S>::STRIDE;
     __shared__ uint4 lds[WAVES][kWave * STRIDE];
     __shared__ unsigned long long bsum[kMaxThresholds];
     __shared__ unsigned int ticket;
@@ -382,48 +373,17 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
     __syncthreads();
     const int lane = lane_id(), wv = wave_in_block_id();
     uint4 *const mine = lds[wv];
-    const int C = (int)score_chunks((int)sizeof(T), V);
+    const int C = (int)row_chunks((int)sizeof(T), V);
     const uint32_t row_bytes = (uint32_t)(V * (int64_t)sizeof(T));
     const int ntiles = (int)((num_vecs + kWave - 1) / kWave);
     const int step = SPLIT == 1 ? (int)gridDim.x * WAVES : (int)gridDim.x;
     const int first = SPLIT == 1 ? (int)blockIdx.x * WAVES + wv : (int)blockIdx.x;
     const int s0 = SPLIT == 1 ? 0 : wv; // this wave's slices: s0, s0 + SPLIT, ...
 
-    // Load i of a slice: chunk g % S of tile row g / S, g = i * 64 + lane.
-    uint32_t offset[S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) {
-        const uint32_t g = (uint32_t)(i * kWave + lane), r = g / S;
-        offset[i] = r * row_bytes + (g - r * S) * 16;
-    }
-    uint4 pre[S];
+    Slice<S> slice;
+    slice.init(row_bytes, lane);
     auto load = [&](int n, int s) { // slice s of the n-th tile from the end
-        const int tile = ntiles - 1 - n;
-        const char *base = reinterpret_cast<const char *>(data) + tile * (int64_t)kWave * (int64_t)row_bytes;
-        const uint32_t at = (uint32_t)(s * S) * 16;
-        if (s + 1 < nslices && tile + 1 < ntiles) { // whole (uniform)
-            base += at;
-#pragma unroll
-            for (int i = 0; i < S; ++i) {
-                const score_chunk_t v = *reinterpret_cast<const score_chunk_t *>(base + offset[i]);
-                pre[i] = make_uint4(v.x, v.y, v.z, v.w);
-            }
-        } else {
-            // rows past the table: the last one again; the row's last chunk ends with it
-            const int64_t left = num_vecs - tile * (int64_t)kWave;
-            const uint32_t last_row = left < kWave ? (uint32_t)left - 1 : kWave - 1;
-            int l = lane;
-            asm volatile("" : "+v"(l)); // computed here, not kept in registers
-#pragma unroll
-            for (int i = 0; i < S; ++i) {
-                const uint32_t g = (uint32_t)(i * kWave + l);
-                uint32_t r = g / S, c = at + (g - r * S) * 16;
-                r = r < last_row ? r : last_row;
-                c = c < row_bytes - 16 ? c : row_bytes - 16;
-                const score_chunk_t v = *reinterpret_cast<const score_chunk_t *>(base + (r * row_bytes + c));
-                pre[i] = make_uint4(v.x, v.y, v.z, v.w);
-            }
-        }
+        slice.load(data, num_vecs, row_bytes, ntiles - 1 - n, ntiles, s, nslices, lane);
     };
 
     auto run = [&](auto na_tag) {
@@ -494,10 +454,7 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
 #pragma unroll
             for (int t = 0; t < NA; ++t) lost[t] = 0;
             for (int s = s0; s < nslices; s += SPLIT) {
-#pragma unroll
-                for (int i = 0; i < S; ++i) {
-                        mine[S % 2 ? i * kWave + lane : (i * (kWave / S) + lane / S) * STRIDE + lane % S] = pre[i];
-                }
+                slice.store(mine, lane);
                 __builtin_amdgcn_wave_barrier();
                 const bool more = s + SPLIT < nslices;
                 const int ns = more ? s + SPLIT : s0;
@@ -594,37 +551,23 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
     select_mask<T>(scores, nt, masks, bitvals, V, mask_out, bitval_out, chosen, threadIdx.x, blockDim.x);
 }
 
-// Launch for nt thresholds (1, or the sweep), N > 0.  As few waves per tile as
-// hold its rows in slices of at most 8 chunks, so a block loads whole rows at
-// once (up to 32 chunks; 512 bytes of each row beyond); 16 waves where rows of
-// more than 1 KB are so few that their tiles leave CUs idle (2292 x 741
-// doubles, the whole call: 232 -> 104 us).  Four waves per SIMD fit (100
-// registers); a fifth gave nothing.
+// Launch for nt thresholds (1, or the sweep), N > 0.  Four waves per SIMD fit
+// (100 registers); a fifth gave nothing.
 template <typename T>
 void launch_score_slices(const T *data, int64_t N, int64_t V, const uint32_t *recs, int nt, Sums *sums, const T *masks,
                          const T *bitvals, T *mask, T *bitval, int32_t *chosen, int num_cus, hipStream_t stream)
 {
-    const int64_t C = score_chunks((int)sizeof(T), V), ntiles = (N + kWave - 1) / kWave;
-    auto go = [&](auto nt_tag, auto s_tag, auto split_tag) {
-        constexpr int NT = decltype(nt_tag)::value, S = decltype(s_tag)::value, SPLIT = decltype(split_tag)::value;
-        constexpr int WAVES = SPLIT == 1 ? 4 : SPLIT;
-        const unsigned long long *flagged = sums->flagged;
-        const int64_t blocks = SPLIT == 1 ? (ntiles + 3) / 4 : ntiles, most = (int64_t)num_cus * (SPLIT == 16 ? 1 : 16 / WAVES);
-        hipLaunchKernelGGL((score_slices_kernel<T, NT, S, SPLIT>), dim3((unsigned)(blocks < most ? blocks : most)),
-                           dim3(kWave * WAVES), 0, stream, data, N, V, (int)((C + S - 1) / S), recs, flagged, nt, sums,
-                           masks, bitvals, mask, bitval, chosen);
-    };
-    using std::integral_constant;
+    const int64_t C = row_chunks((int)sizeof(T), V), ntiles = (N + kWave - 1) / kWave;
     auto by_size = [&](auto nt_tag) {
-        if (C <= 5) go(nt_tag, integral_constant<int, 5>(), integral_constant<int, 1>());
-        else if (C <= 8) go(nt_tag, integral_constant<int, 8>(), integral_constant<int, 1>());
-        else if (C <= 10) go(nt_tag, integral_constant<int, 5>(), integral_constant<int, 2>());
-        else if (C <= 14) go(nt_tag, integral_constant<int, 7>(), integral_constant<int, 2>());
-        else if (C <= 16) go(nt_tag, integral_constant<int, 8>(), integral_constant<int, 2>());
-        else if (C <= 20) go(nt_tag, integral_constant<int, 5>(), integral_constant<int, 4>());
-        else if (C <= 28) go(nt_tag, integral_constant<int, 7>(), integral_constant<int, 4>());
-        else if (C <= 64 || ntiles > num_cus * 2) go(nt_tag, integral_constant<int, 8>(), integral_constant<int, 4>());
-        else go(nt_tag, integral_constant<int, 8>(), integral_constant<int, 16>());
+        with_slices(C, ntiles, num_cus, [&](auto s_tag, auto split_tag) {
+            constexpr int NT = decltype(nt_tag)::value, S = decltype(s_tag)::value, SPLIT = decltype(split_tag)::value;
+            constexpr int WAVES = SPLIT == 1 ? 4 : SPLIT;
+            const unsigned long long *flagged = sums->flagged;
+            const int64_t blocks = SPLIT == 1 ? (ntiles + 3) / 4 : ntiles, most = (int64_t)num_cus * (16 / WAVES);
+            hipLaunchKernelGGL((score_slices_kernel<T, NT, S, SPLIT>), dim3((unsigned)(blocks < most ? blocks : most)),
+                               dim3(kWave * WAVES), 0, stream, data, N, V, (int)((C + S - 1) / S), recs, flagged, nt,
+                               sums, masks, bitvals, mask, bitval, chosen);
+        });
     };
     if (nt == 1) by_size(std::integral_constant<int, 1>());
     else by_size(std::integral_constant<int, kSweep>());
@@ -675,7 +618,7 @@ size_t score_recs_bytes(int w, int64_t V, int nt)
     if (w < 4) return 0;
     const int stride = w == 8 ? (nt == 1 ? ScoreRec<uint64_t, 1>::STRIDE : ScoreRec<uint64_t, kSweep>::STRIDE)
                               : (nt == 1 ? ScoreRec<uint32_t, 1>::STRIDE : ScoreRec<uint32_t, kSweep>::STRIDE);
-    return sizeof(uint32_t) * (size_t)(score_chunks(w, V) * 2 * stride);
+    return sizeof(uint32_t) * (size_t)(row_chunks(w, V) * 2 * stride);
 }
 
 PreWorkspace layout(int w, int64_t V, int nt)
