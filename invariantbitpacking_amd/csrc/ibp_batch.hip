@@ -21,7 +21,6 @@
 #include <vector>
 
 #include "ibp_batch.h"
-#include "ibp_fetch_wide.h"
 #include "ibp_internal.h"
 
 namespace ibp {
@@ -37,7 +36,7 @@ __global__ void batch_reset_kernel(unsigned long long *head)
 // is built per item (two loads per lane); keeping it across items would hold
 // registers for the whole loop.
 template <int ROWS, int KINDS>
-__device__ __forceinline__ void run_item(const TaskDev &t, int64_t b, int64_t e, [[maybe_unused]] uint32_t *wide_lds)
+__device__ __forceinline__ void run_item(const TaskDev &t, int64_t b, int64_t e)
 {
     const FetchParams &p = t.p;
     const bool i32 = p.index != nullptr && t.index_bytes == 4;
@@ -45,11 +44,11 @@ __device__ __forceinline__ void run_item(const TaskDev &t, int64_t b, int64_t e,
     if constexpr ((KINDS & kTasksLarge) != 0) {
         if (KINDS == kTasksLarge || kind == kTasksLarge) {
             if (t.elem_bytes == 8) {
-                if (i32) fetch_wide_range<uint64_t, int32_t>(p, b, e, wide_lds);
-                else fetch_wide_range<uint64_t, int64_t>(p, b, e, wide_lds);
+                if (i32) fetch_large_range<uint64_t, int32_t>(p, b, e, 1);
+                else fetch_large_range<uint64_t, int64_t>(p, b, e, 1);
             } else {
-                if (i32) fetch_wide_range<uint32_t, int32_t>(p, b, e, wide_lds);
-                else fetch_wide_range<uint32_t, int64_t>(p, b, e, wide_lds);
+                if (i32) fetch_large_range<uint32_t, int32_t>(p, b, e, 1);
+                else fetch_large_range<uint32_t, int64_t>(p, b, e, 1);
             }
             return;
         }
@@ -83,8 +82,6 @@ __global__ __launch_bounds__(256) void batch_kernel(const TaskDev *__restrict__ 
                                                     unsigned long long *head, int claim, int dynamic)
 {
     __shared__ int64_t first_item[kLdsTasks];
-    // the waves' LDS for wide rows, in launches that hold such a task
-    __shared__ uint32_t wide_lds[(KINDS & kTasksLarge) ? 4 : 1][(KINDS & kTasksLarge) ? kWideLdsWords : 1];
     const int lane = lane_id();
     const bool staged = ntasks <= kLdsTasks;
     if (staged)
@@ -130,7 +127,7 @@ __global__ __launch_bounds__(256) void batch_kernel(const TaskDev *__restrict__ 
             const int64_t b = (item - t.item_begin) * t.rows_per_item;
             int64_t e = b + t.rows_per_item;
             if (e > t.p.n) e = t.p.n;
-            run_item<ROWS, KINDS>(t, b, e, wide_lds[(KINDS & kTasksLarge) ? wave_in_block_id() : 0]);
+            run_item<ROWS, KINDS>(t, b, e);
         }
     }
 }

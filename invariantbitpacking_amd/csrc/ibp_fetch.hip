@@ -40,8 +40,7 @@ int fetch_launch(const FetchParams &p, int elem_bytes, int index_bytes, int impl
         while (rows > 2 && (p.n + rows - 1) / rows < want) rows /= 2;
     }
 #endif
-    // Wider rows of 4- and 8-byte elements: teams of waves (ibp_fetch_wide.h).
-    const bool wide = p.vec_size > kWave && elem_bytes >= 4 && impl != 2 && impl != 3 && impl != 4;
+    const bool wide = impl != 2 && impl != 3 && impl != 4 && fetch_wide_pays(p, layout, elem_bytes);
     int64_t waves_needed = p.vec_size <= kWave ? (p.n + rows - 1) / rows : p.n;
     int64_t grid = nblks > 0 ? nblks : (waves_needed * kWave + block - 1) / block;
     int64_t cap = (int64_t)dev.num_cus * g_blocks_per_cu.load();

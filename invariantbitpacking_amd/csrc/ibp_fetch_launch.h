@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256) void fetch_small_meta_kernel(FetchParams p)
     }
 }
 
-// Rows of more than 64 elements of 1 or 2 bytes (wider elements: ibp_fetch_wide.h).
+// Rows of more than 64 elements that do not go to teams of waves (ibp_fetch_wide.h).
 template <typename T, typename IdxT, int LAYOUT>
 __global__ __launch_bounds__(256) void fetch_large_kernel(FetchParams p)
 {
@@ -95,8 +95,7 @@ __global__ __launch_bounds__(256) void fetch_baseline_kernel(FetchParams p, int 
     }
 }
 
-// Launches the fetch of one table (rows of more than 64 elements: of 1- and
-// 2-byte elements only): layout (kLayout* flags), impl (2/3/4 the
+// Launches the fetch of one table: layout (kLayout* flags), impl (2/3/4 the
 // transfer baselines), rows in flight per wave for rows of <= 64 elements
 // (2/4/8/16 for 4- and 8-byte elements in the slot layout; 8 otherwise).
 template <typename T, typename IdxT, int LAYOUT>
@@ -104,7 +103,7 @@ void launch_meta(const FetchParams &p, int grid, int block, hipStream_t stream)
 {
     if (p.vec_size <= kWave)
         hipLaunchKernelGGL((fetch_small_meta_kernel<T, IdxT, 8, LAYOUT>), dim3(grid), dim3(block), 0, stream, p);
-    else if constexpr (sizeof(T) < 4)
+    else
         hipLaunchKernelGGL((fetch_large_kernel<T, IdxT, LAYOUT>), dim3(grid), dim3(block), 0, stream, p);
 }
 
@@ -136,7 +135,7 @@ int launch_typed(const FetchParams &p, int layout, int impl, int comp_len, int r
         hipLaunchKernelGGL((fetch_baseline_kernel<T, IdxT>), dim3(grid), dim3(block), 0, stream, p, impl, comp_len);
     } else if (p.vec_size <= kWave) {
         launch_slots_small<T, IdxT>(p, rows, grid, block, stream);
-    } else if constexpr (sizeof(T) < 4) {
+    } else {
         hipLaunchKernelGGL((fetch_large_kernel<T, IdxT, kLayoutSlots>), dim3(grid), dim3(block), 0, stream, p);
     }
     IBP_LAUNCH_CHECK();

@@ -23,6 +23,10 @@
 // 4-byte words (40% packed) 70.0 -> 28.9 us (115 MB: 4.0 TB/s; a device copy
 // runs at 5.0), a 4096 x 2752 block of 8-byte words with 16 mask rows 89 -> 44
 // us, 27,000 rows of 99 words with scattered masks 32.6 -> 21.5 us.
+//
+// With a mask row per cluster the team looks through a window of rows and
+// batches those of one mask row (raw rows need none); what is left over goes to
+// a wave per row.
 #pragma once
 
 #include "ibp_fetch_dev.h"
@@ -30,6 +34,7 @@
 namespace ibp {
 
 constexpr int kWideRows = 8;    // rows of a batch, at most
+constexpr int kWideWindow = 64; // rows among which those of one mask row are looked for, at most
 constexpr int kWideSpan = 64;   // chunks whose positions are worked out together
 constexpr int kWideMaxTeam = 8; // waves of a team, at most
 constexpr int kWideSolo = 4;    // waves of a block of one-wave teams
@@ -168,6 +173,7 @@ struct WideRow {
     int64_t row;    // where the stored row starts
     int64_t stored; // its bytes
     int64_t cursor; // the span's first bit in it
+    int64_t out;    // where the output row starts (mask row per cluster)
 };
 
 // The same rows' stretches of a span: a stretch starts a word before the
@@ -377,7 +383,7 @@ struct WideBatch {
                 x1 = bit_select(f1, (x1 & ~m1) | b1, v1);
                 o = W == 8 ? (wide8_t){x1, x0} : (wide8_t){x0, x1};
             }
-            unsigned char *d = out + r * (p.vec_size * W);
+            unsigned char *d = out + ((LAYOUT & kLayoutClustered) ? readlane(me.out, r) : r * (p.vec_size * W));
             if (MODE == kWhole || left == kCols) {
                 wide8_t *e = reinterpret_cast<wide8_t *>(d) + lane;
                 if constexpr (NT) __builtin_nontemporal_store(o, e);
@@ -390,8 +396,8 @@ struct WideBatch {
         }
     }
 
-    // Rows [0, nrows) of the batch (output rows out0, out0 + 1, ...) of mask
-    // row cl: pk, raw: the packed and the raw rows (the others become zero).
+    // Rows [0, nrows) of the batch (output rows out0, out0 + 1, ...; with
+    // clusters me.out) of mask row cl: pk, raw: the packed and the raw rows (the others become zero).
     __device__ __forceinline__ void run(WideRow me, int nrows, uint32_t pk, uint32_t raw, int64_t cl, int64_t out0) const
     {
         const int64_t V = p.vec_size;
@@ -484,76 +490,100 @@ struct WideBatch {
     }
 };
 
-// Output rows [b, e), kWideRows at most, by a team of waves (fetch_wide_batch
-// is called by every wave of the team with the same arguments but slot; team >
-// 1: the waves of a block).
+// Reads the headers of pinned rows in one go before their words are read by
+// chunk (the team waits in run()): their lines then cross PCIe once.
+__device__ __forceinline__ void touch_headers(const FetchParams &p, int w, const WideRow &me, int nrows, int team, int slot)
+{
+    const int64_t words = header_bytes(p.vec_size, w) / 4;
+    for (int t = slot; t < nrows; t += team) {
+        const uint32_t *h = (const uint32_t *)((const unsigned char *)p.comp + readlane(me.row, t));
+        const int64_t n = readlane(me.stored, t) / 4 < words ? readlane(me.stored, t) / 4 : words;
+        for (int64_t i = lane_id(); i < n; i += kWave) {
+            const uint32_t x = h[i];
+            asm volatile("" ::"v"(x)); // the read is the point
+        }
+    }
+}
+
+// Output rows [b, e) by a team of waves (fetch_wide_batch is called by every
+// wave of the team with the same arguments but slot; team > 1: the waves of a
+// block): kWideRows at most, with clusters kWideWindow, and `least` of one mask
+// row make a batch.
 template <typename T, typename IdxT, int LAYOUT, bool NT>
 __device__ __forceinline__ void fetch_wide_batch(const FetchParams &p, int64_t b, int64_t e, int team, int slot,
-                                                 uint32_t *lds)
+                                                 uint32_t *lds, int least = 1)
 {
-    const int nrows = e - b < kWideRows ? (int)(e - b) : kWideRows;
+    constexpr bool CLUSTERED = (LAYOUT & kLayoutClustered) != 0;
+    constexpr int kRows = CLUSTERED ? kWideWindow : kWideRows;
+    const int nrows = e - b < kRows ? (int)(e - b) : kRows;
     // places past the last row stand for row 0 again
-    const int r = (lane_id() & (kWideRows - 1)) < nrows ? lane_id() & (kWideRows - 1) : 0;
+    const int r = (lane_id() & (kRows - 1)) < nrows ? lane_id() & (kRows - 1) : 0;
     const int64_t s = load_index<IdxT>(p.index, b + r);
     const RowMeta m = decode_meta<T, LAYOUT>(p, s, true, load_meta<LAYOUT>(p, s, true));
-    constexpr uint32_t kLow = (1u << kWideRows) - 1;
-    const uint32_t ok = (uint32_t)ballot(m.ok) & kLow, pk = (uint32_t)ballot(m.ok && m.packed) & kLow;
-    if (p.err && slot == 0 && lane_id() == 0) {
-        const int bad = nrows - (int)__builtin_popcount(ok & ((1u << nrows) - 1));
-        if (bad) atomicAdd(p.err, (unsigned long long)bad);
-    }
     WideRow me;
     me.row = m.word * (int64_t)sizeof(T);
     me.stored = m.len * (int64_t)sizeof(T);
     me.cursor = header_bytes(p.vec_size, (int)sizeof(T)) * 8;
-    if (p.host_rows && p.vec_size * (int64_t)sizeof(T) > 2048) {
-        // Each header read in one go before its words are read by chunk (the
-        // team waits in run()): its lines then cross PCIe once.
-        const int64_t words = header_bytes(p.vec_size, (int)sizeof(T)) / 4;
-        for (int t = slot; t < nrows; t += team) {
-            const uint32_t *h = (const uint32_t *)((const unsigned char *)p.comp + readlane(me.row, t));
-            const int64_t n = readlane(me.stored, t) / 4 < words ? readlane(me.stored, t) / 4 : words;
-            for (int64_t w = lane_id(); w < n; w += kWave) {
-                const uint32_t x = h[w];
-                asm volatile("" ::"v"(x)); // the read is the point
-            }
-        }
-    }
+    me.out = 0;
+    if (p.host_rows && p.vec_size * (int64_t)sizeof(T) > 2048) touch_headers(p, (int)sizeof(T), me, nrows, team, slot);
     const WideBatch<T, LAYOUT, NT> batch(p, team, slot, lds);
-    if constexpr ((LAYOUT & kLayoutClustered) == 0) {
+    constexpr uint32_t kLow = (1u << kWideRows) - 1;
+    if constexpr (!CLUSTERED) {
+        const uint32_t ok = (uint32_t)ballot(m.ok) & kLow, pk = (uint32_t)ballot(m.ok && m.packed) & kLow;
+        if (p.err && slot == 0 && lane_id() == 0) {
+            const int bad = nrows - (int)__builtin_popcount(ok & ((1u << nrows) - 1));
+            if (bad) atomicAdd(p.err, (unsigned long long)bad);
+        }
         batch.run(me, nrows, pk, ok & ~pk, 0, b);
     } else {
-        // Stretches of rows of one mask row (each padded with its first row).
-        for (int r0 = 0; r0 < nrows;) {
-            const int cl = readlane(m.cl, r0);
-            const uint32_t other = (uint32_t)ballot(m.cl != cl) & ((1u << nrows) - 1) & ~((1u << r0) - 1);
-            const int r1 = other ? (int)__builtin_ctz(other) : nrows;
-            const int place = lane_id() & (kWideRows - 1);
-            const int from = place < r1 - r0 ? r0 + place : r0;
-            WideRow part = me;
-            part.row = (int64_t)shfl((uint64_t)me.row, from);
-            part.stored = (int64_t)shfl((uint64_t)me.stored, from);
-            const uint32_t part_ok = (uint32_t)ballot((ok >> from) & 1) & kLow;
-            const uint32_t part_pk = (uint32_t)ballot((pk >> from) & 1) & kLow;
-            batch.run(part, r1 - r0, part_pk, part_ok & ~part_pk, cl, b + r0);
-            r0 = r1;
+        // Batches of the window's rows of one mask row, wherever they stand in it
+        const uint64_t in = nrows == kWave ? ~0ull : (1ull << nrows) - 1;
+        const uint64_t pk = ballot(m.packed);
+        uint64_t left = ballot(m.ok) & in;
+        if (uint64_t bad = in & ~left) { // rows that are refused: zeros
+            if (p.err && slot == 0 && lane_id() == 0) atomicAdd(p.err, (unsigned long long)__builtin_popcountll(bad));
+            for (; bad; bad &= bad - 1) {
+                T *dst = (T *)p.out + (b + __builtin_ctzll(bad)) * p.vec_size;
+                for (int64_t k = slot * kWave + lane_id(); k < p.vec_size; k += team * kWave) dst[k] = T(0);
+            }
+        }
+        // (fewer than `least` of them go to a wave each, below)
+        uint64_t single = 0;
+        const int key = m.packed ? m.cl : -1; // raw rows need no mask row
+        while (left) {
+            const int kind = readlane(key, __builtin_ctzll(left)), cl = kind < 0 ? 0 : kind;
+            uint64_t alike = ballot(key == kind) & left;
+            left &= ~alike;
+            while (__builtin_popcountll(alike) >= least) {
+                // place k of the batch: the k-th of them; places past the last stand for the first
+                const int place = lane_id() & (kWideRows - 1);
+                int from = __builtin_ctzll(alike), n = 0;
+#pragma unroll
+                for (int k = 0; k < kWideRows; ++k) {
+                    if (!alike) break; // uniform
+                    const int at = __builtin_ctzll(alike);
+                    alike &= alike - 1;
+                    from = place == k ? at : from;
+                    ++n;
+                }
+                WideRow part = me;
+                part.row = (int64_t)shfl((uint64_t)me.row, from);
+                part.stored = (int64_t)shfl((uint64_t)me.stored, from);
+                part.out = (int64_t)from * (p.vec_size * (int64_t)sizeof(T));
+                const uint32_t part_pk = (uint32_t)ballot((pk >> from) & 1) & kLow;
+                batch.run(part, n, part_pk, kLow & ~part_pk, cl, b);
+            }
+            single |= alike;
+        }
+        for (int k = 0; single; ++k, single &= single - 1) {
+            const int at = __builtin_ctzll(single);
+            if (k % team == slot) fetch_large_row_from<T, LAYOUT>(p, b + at, readlane(s, at));
         }
     }
 }
 
-// Output rows [b, e) by one wave.
-template <typename T, typename IdxT, int LAYOUT = kLayoutSlots>
-__device__ __forceinline__ void fetch_wide_range(const FetchParams &p, int64_t b, int64_t e, uint32_t *lds)
-{
-    for (int64_t i = b; i < e; i += kWideRows) {
-        const int64_t to = e < i + kWideRows ? e : i + kWideRows;
-        if (rows_fill_lines(p.vec_size, (int)sizeof(T)))
-            fetch_wide_batch<T, IdxT, LAYOUT, true>(p, i, to, 1, 0, lds);
-        else
-            fetch_wide_batch<T, IdxT, LAYOUT, false>(p, i, to, 1, 0, lds);
-    }
-}
-
+// Whether teams of waves are the faster way (else a wave per row).
+bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes);
 // The plain fetch's launch for rows of more than 64 elements of 4 or 8 bytes
 // (ibp_fetch_wide.hip); nblks <= 0: a grid for the rows.
 int fetch_wide_launch(const FetchParams &p, int layout, int elem_bytes, int index_bytes, int nblks,
