@@ -1574,7 +1574,13 @@ int pack_typed(PackParams p, hipStream_t stream)
 template <typename T>
 int pack_width(const PackParams &p, int index_bytes, hipStream_t s)
 {
-    if (sizeof(T) >= 4 && p.V > kWave && p.V * (int64_t)sizeof(T) <= kPackWideMaxBytes)
+    // Teams of waves per row (ibp_pack_wide.hip): rows of 512 columns and more
+    // whatever their number (500 to 60,000 rows of 600 words: 28 to 192 us,
+    // against 45 to 288 here, the copy of the table included), narrower ones
+    // from 32768 rows on (60,000 rows of 65 words 59 against 81, 16,000 rows 40
+    // against 34).
+    if (sizeof(T) >= 4 && p.V > kWave && p.V * (int64_t)sizeof(T) <= kPackWideMaxBytes &&
+        (p.V >= 512 || p.n >= 32768))
         return pack_wide_launch(p, (int)sizeof(T), index_bytes, s);
     const bool i32 = p.index && index_bytes == 4;
     if (p.offsets)

@@ -1,5 +1,5 @@
-"""GPU parity of the fetch by teams of waves where it is chosen by size: many
-rows of 65 to 511 columns, and windows of rows of several mask rows (batches of
+"""GPU parity of the fetch and pack by teams of waves where they are chosen by
+size: many rows of 65 to 511 columns, and windows of rows of several mask rows (batches of
 one mask row, raw rows, single rows, refused rows), in every window size."""
 import numpy as np
 import pytest
@@ -82,3 +82,23 @@ def test_windows_of_mask_rows(ibp, oracle, w, v, k, n):
     bad = rng.choice(203, size=3, replace=False) if k > 1 else None
     print("windows", w, v, k, n, flush=True)
     fetch_all(ibp, oracle, x.view(dt), mask.view(dt), bitval.view(dt), idx, cl, bad)
+
+
+@pytest.mark.parametrize("w,v", [(4, 65), (4, 129), (8, 65), (8, 128)])
+def test_pack_of_many_rows(ibp, oracle, w, v):
+    rng = np.random.default_rng(10 * w + v)
+    dt = np.dtype("i%d" % w)
+    mask = np.stack([masks_of("mixed", v, w, rng) for _ in range(2)])
+    bitval = rng.integers(0, 2 ** 63, size=mask.shape, dtype=np.uint64).astype(mask.dtype) & mask
+    n = 32768 + 33
+    cl = (rng.random(n) < 0.3).astype(np.int32)
+    x = np.where(cl[:, None] == 0, rows_for(n, mask[0], bitval[0], rng), rows_for(n, mask[1], bitval[1], rng)).view(dt)
+    m, b = mask.view(dt), bitval.view(dt)
+    print("pack teams", w, v, flush=True)
+    for mm, bb, kw, kd in ((m[0].copy(), b[0].copy(), {}, {}),
+                           (m, b, {"clusters": cl}, {"clusters": torch.from_numpy(cl).cuda()})):
+        comp, bm = oracle.compress(x, mm, bb, **kw)
+        t = torch.from_numpy(x.copy()).cuda()
+        got = ibp.compress_inplace(t, torch.from_numpy(mm).cuda(), torch.from_numpy(bb).cuda(), **kd)
+        assert np.array_equal(got.cpu().numpy().view(np.uint32), bm.view(np.uint32))
+        assert np.array_equal(t.cpu().numpy().view(comp.dtype), comp)
