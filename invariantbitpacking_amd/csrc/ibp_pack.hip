@@ -1509,7 +1509,8 @@ int pack_typed(PackParams p, hipStream_t stream)
         // group, with slot buffers in LDS when four or more fit one CU's LDS
         // (as many waves as fit, up to 16), else 16 waves with buffers in
         // device memory.
-        const int64_t lds_cu = 160 * 1024;
+        // (the kernel's own variable in LDS left out)
+        const int64_t lds_cu = 160 * 1024 - 64;
         const bool lds = buf_bytes * 4 <= lds_cu;
         int wpb = lds ? (int)((buf_bytes * 8 <= lds_budget ? lds_budget : lds_cu) / buf_bytes) : 16;
         if (wpb > 16) wpb = 16;
