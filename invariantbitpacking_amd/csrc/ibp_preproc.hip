@@ -27,8 +27,13 @@ constexpr int kSweep = 7; // thresholds of the sweep: 0.70, 0.75, ... 1.00
 // Sums that the kernels of one call add to, cleared by the first of them.
 struct Sums {
     unsigned long long score[kMaxThresholds]; // bits saved
-    unsigned long long flagged[kMaxThresholds]; // bits of all columns' masks
     unsigned int blocks; // scoring blocks that are done
+    // Bits of all columns' masks: kCopies partial sums in lines of their own
+    // (one line for the 512 blocks of a table of 1024 columns: 47 us of atomics)
+    static constexpr int kCopies = 16;
+    struct alignas(128) Flagged {
+        unsigned long long t[kMaxThresholds];
+    } flagged[kCopies];
 };
 __device__ __forceinline__ void clear_sums(Sums *sums)
 {
@@ -210,7 +215,7 @@ __global__ __launch_bounds__(1024) void masks_kernel(const int32_t *part, int64_
             masks[t * V + j] = m[t];
             bitvals[t * V + j] = v;
         }
-        if (lane == 0) atomicAdd(&total->flagged[t], (unsigned long long)__builtin_popcountll(all));
+        if (lane == 0) atomicAdd(&total->flagged[blockIdx.x % Sums::kCopies].t[t], (unsigned long long)__builtin_popcountll(all));
     }
     if constexpr (sizeof(T) >= 4) {
         if (recs && lane < COLS && j < V) {
@@ -360,7 +365,7 @@ __global__ void clear_kernel(Sums *sums) { clear_sums(sums); }
 template <typename T, int NT, int S, int SPLIT>
 __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_kernel(
     const T *__restrict__ data, int64_t num_vecs, int64_t V, int nslices, const uint32_t *__restrict__ recs,
-    const unsigned long long *__restrict__ flagged, int nt, Sums *sums, const T *__restrict__ masks,
+    const Sums::Flagged *__restrict__ flagged, int nt, Sums *sums, const T *__restrict__ masks,
     const T *__restrict__ bitvals, T *mask_out, T *bitval_out, int32_t *chosen)
 {
     using R = ScoreRec<T, NT>;
@@ -386,13 +391,20 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
         slice.load(data, num_vecs, row_bytes, ntiles - 1 - n, ntiles, s, nslices, lane);
     };
 
+    uint32_t all[NT]; // bits of all columns' masks
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        all[t] = 0;
+        for (int k = 0; k < Sums::kCopies; ++k) all[t] += (uint32_t)flagged[k].t[t];
+    }
+
     auto run = [&](auto na_tag) {
         constexpr int NA = decltype(na_tag)::value;
         uint32_t total[NA];
         unsigned long long saved[NA];
 #pragma unroll
         for (int t = 0; t < NA; ++t) {
-            total[t] = (uint32_t)flagged[t];
+            total[t] = all[t];
             asm volatile("" : "+v"(total[t])); // the scalar registers are for the units
             saved[t] = 0;
         }
@@ -523,7 +535,7 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
     int na = 0;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
-        if (t < nt && flagged[t]) na = t + 1;
+        if (t < nt && all[t]) na = t + 1;
     if constexpr (NT == 1) {
         if (na) run(std::integral_constant<int, 1>());
     } else {
@@ -562,7 +574,7 @@ void launch_score_slices(const T *data, int64_t N, int64_t V, const uint32_t *re
         with_slices(C, ntiles, num_cus, [&](auto s_tag, auto split_tag) {
             constexpr int NT = decltype(nt_tag)::value, S = decltype(s_tag)::value, SPLIT = decltype(split_tag)::value;
             constexpr int WAVES = SPLIT == 1 ? 4 : SPLIT;
-            const unsigned long long *flagged = sums->flagged;
+            const Sums::Flagged *flagged = sums->flagged;
             const int64_t blocks = SPLIT == 1 ? (ntiles + 3) / 4 : ntiles, most = (int64_t)num_cus * (16 / WAVES);
             hipLaunchKernelGGL((score_slices_kernel<T, NT, S, SPLIT>), dim3((unsigned)(blocks < most ? blocks : most)),
                                dim3(kWave * WAVES), 0, stream, data, N, V, (int)((C + S - 1) / S), recs, flagged, nt,
