@@ -20,8 +20,8 @@
 // load depends on another chunk's payload, the loads of up to eight rows are
 // in flight per wave, and a column's layout is worked out once per batch: 70
 // operations.  Measured against the wave per row: 20,000 random 4 KiB rows of
-// 4-byte words (40% packed) 70.0 -> 28.9 us (115 MB: 4.0 TB/s; a device copy
-// runs at 5.0), a 4096 x 2752 block of 8-byte words with 16 mask rows 89 -> 44
+// 4-byte words (40% packed) 70.0 -> 31.1 us (115 MB: 3.7 TB/s; a device copy
+// runs at 5.0), a 4096 x 2752 block of 8-byte words with 16 mask rows 92 -> 48
 // us, 27,000 rows of 99 words with scattered masks 32.6 -> 21.5 us.
 //
 // With a mask row per cluster the team looks through a window of rows and
@@ -46,6 +46,7 @@ constexpr int kWideLdsWords = kWideRows * kWideStride;
 typedef uint32_t wide8_t __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t wide12_t __attribute__((ext_vector_type(3), aligned(4)));
 typedef uint32_t wide16_t __attribute__((ext_vector_type(4), aligned(8)));
+typedef uint32_t raw16_t __attribute__((ext_vector_type(4), aligned(4)));
 
 // A lane's 8 bytes of mask or bitval in a chunk, as the half that comes first
 // in the stream and the other; `left` of the chunk's columns are in the row
@@ -396,6 +397,44 @@ struct WideBatch {
         }
     }
 
+    // A batch without a packed row: its rows as they are stored (raw) or zero,
+    // in pieces of 4 KiB spread over the team, four 16-byte loads in flight per
+    // lane (4096 raw rows of 1024 and 2752 doubles by chunks 1431 GB/s, so 2165).
+    __device__ __forceinline__ void copy_rows(const WideRow &me, int nrows, uint32_t raw, unsigned char *out) const
+    {
+        const int64_t bytes = p.vec_size * W;
+        int turn = 0;
+        for (int r = 0; r < nrows; ++r) {
+            const unsigned char *src = comp + readlane(me.row, r);
+            unsigned char *dst = out + ((LAYOUT & kLayoutClustered) ? readlane(me.out, r) : r * bytes);
+            const bool stored = (raw >> r) & 1;
+            for (int64_t at = 0; at < bytes; at += 4096, turn = turn + 1 == team ? 0 : turn + 1) {
+                if (turn != slot) continue; // uniform
+                const int64_t o = at + fresh_lane() * 16;
+                wide16_t v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    v[u] = (wide16_t){0u, 0u, 0u, 0u};
+                    if (stored && o + u * 1024 + 16 <= bytes)
+                        v[u] = *reinterpret_cast<const raw16_t *>(src + o + u * 1024);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int64_t k = o + u * 1024;
+                    if (k + 16 <= bytes) {
+                        raw16_t *e = reinterpret_cast<raw16_t *>(dst + k);
+                        if constexpr (NT) __builtin_nontemporal_store((raw16_t)v[u], e);
+                        else *e = v[u];
+                    } else { // the row's last words
+                        for (int64_t i = k; i < bytes; i += 4)
+                            *reinterpret_cast<uint32_t *>(dst + i) =
+                                stored ? *reinterpret_cast<const uint32_t *>(src + i) : 0u;
+                    }
+                }
+            }
+        }
+    }
+
     // Rows [0, nrows) of the batch (output rows out0, out0 + 1, ...; with
     // clusters me.out) of mask row cl: pk, raw: the packed and the raw rows (the others become zero).
     __device__ __forceinline__ void run(WideRow me, int nrows, uint32_t pk, uint32_t raw, int64_t cl, int64_t out0) const
@@ -405,6 +444,10 @@ struct WideBatch {
         const int64_t nchunks = (V + kCols - 1) / kCols;
         const uint32_t live = (1u << nrows) - 1;
         unsigned char *out = (unsigned char *)p.out + out0 * (V * W);
+        if (!pk && !p.host_rows) { // uniform for the team (over PCIe by chunks: 57 against 55 GB/s)
+            copy_rows(me, nrows, raw, out);
+            return;
+        }
         auto cols_left = [&](int64_t c) { return V - c * kCols < kCols ? (int)(V - c * kCols) : kCols; };
         for (int64_t c0 = 0; c0 < nchunks; c0 += kWideSpan) {
             const int nc = nchunks - c0 < kWideSpan ? (int)(nchunks - c0) : kWideSpan;
@@ -490,12 +533,14 @@ struct WideBatch {
     }
 };
 
-// Reads the headers of pinned rows in one go before their words are read by
+// Reads the headers of packed pinned rows in one go before their words are read by
 // chunk (the team waits in run()): their lines then cross PCIe once.
-__device__ __forceinline__ void touch_headers(const FetchParams &p, int w, const WideRow &me, int nrows, int team, int slot)
+__device__ __forceinline__ void touch_headers(const FetchParams &p, int w, const WideRow &me, uint64_t packed, int nrows, int team,
+                                              int slot)
 {
     const int64_t words = header_bytes(p.vec_size, w) / 4;
     for (int t = slot; t < nrows; t += team) {
+        if (!((packed >> t) & 1)) continue; // uniform
         const uint32_t *h = (const uint32_t *)((const unsigned char *)p.comp + readlane(me.row, t));
         const int64_t n = readlane(me.stored, t) / 4 < words ? readlane(me.stored, t) / 4 : words;
         for (int64_t i = lane_id(); i < n; i += kWave) {
@@ -525,7 +570,8 @@ __device__ __forceinline__ void fetch_wide_batch(const FetchParams &p, int64_t b
     me.stored = m.len * (int64_t)sizeof(T);
     me.cursor = header_bytes(p.vec_size, (int)sizeof(T)) * 8;
     me.out = 0;
-    if (p.host_rows && p.vec_size * (int64_t)sizeof(T) > 2048) touch_headers(p, (int)sizeof(T), me, nrows, team, slot);
+    if (p.host_rows && p.vec_size * (int64_t)sizeof(T) > 2048)
+        touch_headers(p, (int)sizeof(T), me, ballot(m.ok && m.packed), nrows, team, slot);
     const WideBatch<T, LAYOUT, NT> batch(p, team, slot, lds);
     constexpr uint32_t kLow = (1u << kWideRows) - 1;
     if constexpr (!CLUSTERED) {
