@@ -21,12 +21,12 @@
 // in flight per wave, and a column's layout is worked out once per batch: 70
 // operations.  Measured against the wave per row: 20,000 random 4 KiB rows of
 // 4-byte words (40% packed) 70.0 -> 31.1 us (115 MB: 3.7 TB/s; a device copy
-// runs at 5.0), a 4096 x 2752 block of 8-byte words with 16 mask rows 92 -> 48
-// us, 27,000 rows of 99 words with scattered masks 32.6 -> 21.5 us.
+// runs at 5.0), a 4096 x 2752 block of 8-byte words whose rows share one of 16
+// mask rows 92 -> 47 us, 27,000 rows of 99 words with scattered masks 32.6 -> 21.5 us.
 //
 // With a mask row per cluster the team looks through a window of rows and
-// batches those of one mask row (raw rows need none); what is left over goes to
-// a wave per row.
+// batches those of one mask row (raw rows need none) where they are most of it;
+// the others go to a wave per row, or to two.
 #pragma once
 
 #include "ibp_fetch_dev.h"
@@ -174,7 +174,7 @@ struct WideRow {
     int64_t row;    // where the stored row starts
     int64_t stored; // its bytes
     int64_t cursor; // the span's first bit in it
-    int64_t out;    // where the output row starts (mask row per cluster)
+    int out;        // its output row, from the batch's first one (mask row per cluster)
 };
 
 // The same rows' stretches of a span: a stretch starts a word before the
@@ -185,9 +185,12 @@ struct WideStretch {
     uint32_t q;    // chunk: the bit before its first one
 };
 
-// NT: the store policy (rows_fill_lines).
-template <typename T, int LAYOUT, bool NT>
+// NT: the store policy (rows_fill_lines).  SUB: rows unpacked together, at most:
+// 8, 4, or 1 (batches are single rows).  LOCKSTEP: teams of one block run rows
+// of their own together, so every wave passes every barrier, whatever its row.
+template <typename T, int LAYOUT, bool NT, int SUB, bool LOCKSTEP = false>
 struct WideBatch {
+    static constexpr bool ONE = SUB == 1;
     static constexpr int W = (int)sizeof(T);
     static constexpr int kCols = 512 / W; // columns of a chunk
     enum : int { kAny, kFast, kWhole };
@@ -321,13 +324,13 @@ struct WideBatch {
         return ((uint64_t)hi << 32) | lo;
     }
 
-    // Phase C for rows [r0, r0 + SUB) of the batch, chunk c: m, b the
+    // Phase C for rows [r0, r0 + N) of the batch, chunk c: m, b the
     // column's mask and bitval halves, w their codes (TWO: the two-run
     // form); pk, raw, live: the rows'
     // kinds; out: the chunk of output row 0.  kAny: rows of any kind.
     // kFast: every row is packed and its windows lie inside the stored row;
     // kWhole: and the chunk is whole.
-    template <int MODE, bool TWO, int SUB, int r0>
+    template <int MODE, bool TWO, int N, int r0>
     __device__ __forceinline__ void unpack_rows(const WideRow &me, const WideStretch &st, uint32_t pk,
                                                 uint32_t raw, uint32_t live, uint32_t inside, unsigned char *out,
                                                 int64_t c, int left, uint32_t flags, const WideCode &w0,
@@ -340,10 +343,10 @@ struct WideBatch {
         const int words = left * (W / 4);
         // bits of this lane's columns
         const int full = MODE == kWhole || 2 * lane + 2 <= words ? 64 : 2 * lane < words ? 32 : 0;
-        Window win[SUB];
-        uint32_t q[SUB], f[SUB];
+        Window win[N];
+        uint32_t q[N], f[N];
 #pragma unroll
-        for (int u = 0; u < SUB; ++u) {
+        for (int u = 0; u < N; ++u) {
             const int r = r0 + u;
             win[u] = {0u, 0u, 0u, 0u};
             q[u] = f[u] = 0;
@@ -370,7 +373,7 @@ struct WideBatch {
             }
         }
 #pragma unroll
-        for (int u = 0; u < SUB; ++u) {
+        for (int u = 0; u < N; ++u) {
             const int r = r0 + u;
             if (MODE != kWhole && !((live >> r) & 1)) continue; // uniform
             wide8_t o = {win[u].d0, win[u].d1};
@@ -384,7 +387,7 @@ struct WideBatch {
                 x1 = bit_select(f1, (x1 & ~m1) | b1, v1);
                 o = W == 8 ? (wide8_t){x1, x0} : (wide8_t){x0, x1};
             }
-            unsigned char *d = out + ((LAYOUT & kLayoutClustered) ? readlane(me.out, r) : r * (p.vec_size * W));
+            unsigned char *d = out + ((LAYOUT & kLayoutClustered) ? readlane(me.out, r) : r) * (p.vec_size * W);
             if (MODE == kWhole || left == kCols) {
                 wide8_t *e = reinterpret_cast<wide8_t *>(d) + lane;
                 if constexpr (NT) __builtin_nontemporal_store(o, e);
@@ -406,7 +409,7 @@ struct WideBatch {
         int turn = 0;
         for (int r = 0; r < nrows; ++r) {
             const unsigned char *src = comp + readlane(me.row, r);
-            unsigned char *dst = out + ((LAYOUT & kLayoutClustered) ? readlane(me.out, r) : r * bytes);
+            unsigned char *dst = out + ((LAYOUT & kLayoutClustered) ? readlane(me.out, r) : r) * bytes;
             const bool stored = (raw >> r) & 1;
             for (int64_t at = 0; at < bytes; at += 4096, turn = turn + 1 == team ? 0 : turn + 1) {
                 if (turn != slot) continue; // uniform
@@ -444,36 +447,42 @@ struct WideBatch {
         const int64_t nchunks = (V + kCols - 1) / kCols;
         const uint32_t live = (1u << nrows) - 1;
         unsigned char *out = (unsigned char *)p.out + out0 * (V * W);
-        if (!pk && !p.host_rows) { // uniform for the team (over PCIe by chunks: 57 against 55 GB/s)
+        const bool copied = !pk && !p.host_rows; // uniform for the team (over PCIe by chunks: 57 against 55 GB/s)
+        if (copied) {
             copy_rows(me, nrows, raw, out);
-            return;
+            if constexpr (!LOCKSTEP) return;
         }
         auto cols_left = [&](int64_t c) { return V - c * kCols < kCols ? (int)(V - c * kCols) : kCols; };
         for (int64_t c0 = 0; c0 < nchunks; c0 += kWideSpan) {
             const int nc = nchunks - c0 < kWideSpan ? (int)(nchunks - c0) : kWideSpan;
-            if (pk) { // uniform for the team
+            if (LOCKSTEP || pk) { // uniform for the team
                 sync(); // the positions before these have been read
-                for (int k = slot; k < nc; k += team) {
+                for (int k = pk ? slot : nc; k < nc; k += team) {
                     const int lane = fresh_lane();
                     const int left = cols_left(c0 + k);
                     uint32_t m0, m1;
                     load_wide_cols<T>(mask + (c0 + k) * kCols, left, m0, m1);
                     const uint32_t flags = load_flags(me, c0 + k, pk);
                     const int s0 = __builtin_popcount(m0), s1 = __builtin_popcount(m1);
-                    int x[kWideRows], z0, z1;
+                    if constexpr (ONE) {
+                        const int z = wave_sum(lane_saved(lane, lane_flags(lane, flags, 0), s0, s1));
+                        if (lane == 0) lds[k] = (uint32_t)(left * W * 8 - z);
+                    } else {
+                        int x[kWideRows], z0, z1;
 #pragma unroll
-                    for (int r = 0; r < kWideRows; ++r) {
-                        x[r] = lane_saved(lane, lane_flags(lane, flags, r), s0, s1);
-                    }
-                    wave_sum8(x, z0, z1);
-                    if ((lane & 15) == 15) {
-                        uint32_t *t = lds + 2 * (lane >> 4) * kWideStride + k;
-                        t[0] = (uint32_t)(left * W * 8 - z0);
-                        t[kWideStride] = (uint32_t)(left * W * 8 - z1);
+                        for (int r = 0; r < kWideRows; ++r) {
+                            x[r] = lane_saved(lane, lane_flags(lane, flags, r), s0, s1);
+                        }
+                        wave_sum8(x, z0, z1);
+                        if ((lane & 15) == 15) {
+                            uint32_t *t = lds + 2 * (lane >> 4) * kWideStride + k;
+                            t[0] = (uint32_t)(left * W * 8 - z0);
+                            t[kWideStride] = (uint32_t)(left * W * 8 - z1);
+                        }
                     }
                 }
                 sync();
-                for (int r = slot; r < kWideRows; r += team) {
+                for (int r = pk ? slot : kWideRows; r < (ONE ? 1 : kWideRows); r += team) {
                     uint32_t *t = lds + r * kWideStride;
                     const int x = lane < nc ? (int)t[lane] : 0;
                     const int incl = wave_incl_scan(x);
@@ -482,7 +491,8 @@ struct WideBatch {
                 }
                 sync();
             }
-            const uint32_t *mine = lds + (lane & 7) * kWideStride; // this lane's row's positions
+            if (LOCKSTEP && (copied || nrows == 0)) continue;
+            const uint32_t *mine = lds + (ONE ? 0 : (lane & 7) * kWideStride); // this lane's row's positions
             WideStretch st;
             const int64_t at = (me.cursor >> (W == 8 ? 6 : 5)) * W - W;
             const int64_t room = me.stored - at;
@@ -514,17 +524,17 @@ struct WideBatch {
                         me, st, pk, raw, live, inside, out + c * 512, c, left, flags, w0, w1, m0, m1, b0, b1);
                 };
                 auto rows = [&](auto mode, auto form) {
-                    constexpr int kSub = decltype(mode)::value == kWhole && decltype(form)::value ? 8 : 4;
+                    constexpr int kSub = SUB < 8 || (decltype(mode)::value == kWhole && decltype(form)::value) ? SUB : 4;
                     go(mode, form, Int<kSub>(), Int<0>());
-                    if constexpr (kSub < kWideRows)
-                        if (nrows > kSub) go(mode, form, Int<kSub>(), Int<kSub>());
+                    if constexpr (kSub == 4)
+                        if (nrows > 4) go(mode, form, Int<kSub>(), Int<4>());
                 };
                 auto go_mode = [&](auto mode) {
                     if (two) rows(mode, std::true_type());
                     else rows(mode, std::false_type());
                 };
                 const bool fast = (pk & inside & 0xffu) == 0xffu;
-                if (fast && nrows == kWideRows && left == kCols) go_mode(Int<kWhole>());
+                if (fast && (ONE || nrows == kWideRows) && left == kCols) go_mode(Int<kWhole>());
                 else if (fast) go_mode(Int<kFast>());
                 else go_mode(Int<kAny>());
             }
@@ -532,6 +542,17 @@ struct WideBatch {
         }
     }
 };
+
+template <typename T>
+__device__ __forceinline__ WideRow wide_row(const FetchParams &p, const RowMeta &m)
+{
+    WideRow r;
+    r.row = m.word * (int64_t)sizeof(T);
+    r.stored = m.len * (int64_t)sizeof(T);
+    r.cursor = header_bytes(p.vec_size, (int)sizeof(T)) * 8;
+    r.out = 0;
+    return r;
+}
 
 // Reads the headers of packed pinned rows in one go before their words are read by
 // chunk (the team waits in run()): their lines then cross PCIe once.
@@ -550,80 +571,166 @@ __device__ __forceinline__ void touch_headers(const FetchParams &p, int w, const
     }
 }
 
-// Output rows [b, e) by a team of waves (fetch_wide_batch is called by every
-// wave of the team with the same arguments but slot; team > 1: the waves of a
-// block): kWideRows at most, with clusters kWideWindow, and `least` of one mask
-// row make a batch.
+// Output rows [b, e) by a team of waves (called by every wave of the team with
+// the same arguments but slot; team > 1: the waves of a block): kWideRows at
+// most make a batch.
 template <typename T, typename IdxT, int LAYOUT, bool NT>
 __device__ __forceinline__ void fetch_wide_batch(const FetchParams &p, int64_t b, int64_t e, int team, int slot,
-                                                 uint32_t *lds, int least = 1)
+                                                 uint32_t *lds)
 {
-    constexpr bool CLUSTERED = (LAYOUT & kLayoutClustered) != 0;
-    constexpr int kRows = CLUSTERED ? kWideWindow : kWideRows;
-    const int nrows = e - b < kRows ? (int)(e - b) : kRows;
+    const int nrows = e - b < kWideRows ? (int)(e - b) : kWideRows;
     // places past the last row stand for row 0 again
-    const int r = (lane_id() & (kRows - 1)) < nrows ? lane_id() & (kRows - 1) : 0;
+    const int r = (lane_id() & (kWideRows - 1)) < nrows ? lane_id() & (kWideRows - 1) : 0;
     const int64_t s = load_index<IdxT>(p.index, b + r);
     const RowMeta m = decode_meta<T, LAYOUT>(p, s, true, load_meta<LAYOUT>(p, s, true));
-    WideRow me;
-    me.row = m.word * (int64_t)sizeof(T);
-    me.stored = m.len * (int64_t)sizeof(T);
-    me.cursor = header_bytes(p.vec_size, (int)sizeof(T)) * 8;
-    me.out = 0;
+    const WideRow me = wide_row<T>(p, m);
     if (p.host_rows && p.vec_size * (int64_t)sizeof(T) > 2048)
         touch_headers(p, (int)sizeof(T), me, ballot(m.ok && m.packed), nrows, team, slot);
-    const WideBatch<T, LAYOUT, NT> batch(p, team, slot, lds);
+    const WideBatch<T, LAYOUT, NT, (LAYOUT & kLayoutClustered) ? 1 : 8> batch(p, team, slot, lds);
     constexpr uint32_t kLow = (1u << kWideRows) - 1;
-    if constexpr (!CLUSTERED) {
-        const uint32_t ok = (uint32_t)ballot(m.ok) & kLow, pk = (uint32_t)ballot(m.ok && m.packed) & kLow;
-        if (p.err && slot == 0 && lane_id() == 0) {
-            const int bad = nrows - (int)__builtin_popcount(ok & ((1u << nrows) - 1));
-            if (bad) atomicAdd(p.err, (unsigned long long)bad);
+    const uint32_t ok = (uint32_t)ballot(m.ok) & kLow, pk = (uint32_t)ballot(m.ok && m.packed) & kLow;
+    if (p.err && slot == 0 && lane_id() == 0) {
+        const int bad = nrows - (int)__builtin_popcount(ok & ((1u << nrows) - 1));
+        if (bad) atomicAdd(p.err, (unsigned long long)bad);
+    }
+    // (with clusters: one row)
+    batch.run(me, nrows, pk, ok & ~pk, (LAYOUT & kLayoutClustered) ? readlane(m.cl, 0) : 0, b);
+}
+
+// With a mask row per cluster: the rows [b, e) of a window, lane r: row r.
+template <typename T>
+struct WideWindow {
+    RowMeta m;
+    int key;     // what rows of one batch share: the mask row, -1 for raw rows, which need none; -2: refused
+    uint64_t ok; // the rows that are not refused
+    int nrows;
+
+    template <typename IdxT, int LAYOUT>
+    __device__ __forceinline__ void load(const FetchParams &p, int64_t b, int64_t e)
+    {
+        nrows = (int)(e - b);
+        const int r = lane_id() < nrows ? lane_id() : 0;
+        const int64_t s = load_index<IdxT>(p.index, b + r);
+        m = decode_meta<T, LAYOUT>(p, s, true, load_meta<LAYOUT>(p, s, true));
+        key = !m.ok ? -2 : m.packed ? m.cl : -1;
+        count();
+    }
+    __device__ __forceinline__ void count()
+    {
+        ok = ballot(key != -2) & (nrows == kWave ? ~0ull : (1ull << nrows) - 1);
+    }
+    // Row r, which is the same for the whole wave.
+    __device__ __forceinline__ RowMeta row(int r) const
+    {
+        RowMeta me;
+        me.word = readlane(m.word, r);
+        me.len = readlane(m.len, r);
+        me.cl = readlane(m.cl, r);
+        me.ok = (ok >> r) & 1;
+        me.packed = me.ok && readlane(key, r) >= 0;
+        return me;
+    }
+    // The rows that one batch may hold beside row r, which is not refused.
+    __device__ __forceinline__ uint64_t alike(int r) const { return ballot(key == readlane(key, r)) & ok; }
+    // The rows that a team takes: those of one mask row and the raw ones, if
+    // they are `least` at least; else none.
+    __device__ __forceinline__ uint64_t batched(int least) const
+    {
+        const uint64_t raw = ballot(key == -1) & ok;
+        uint64_t left = ok & ~raw;
+        const int nraw = __builtin_popcountll(raw);
+        while (__builtin_popcountll(left) + nraw >= least) { // uniform
+            if (!left) return raw;
+            const uint64_t same = alike(__builtin_ctzll(left));
+            if (__builtin_popcountll(same) + nraw >= least) return same | raw;
+            left &= ~same;
         }
-        batch.run(me, nrows, pk, ok & ~pk, 0, b);
-    } else {
-        // Batches of the window's rows of one mask row, wherever they stand in it
-        const uint64_t in = nrows == kWave ? ~0ull : (1ull << nrows) - 1;
-        const uint64_t pk = ballot(m.packed);
-        uint64_t left = ballot(m.ok) & in;
-        if (uint64_t bad = in & ~left) { // rows that are refused: zeros
-            if (p.err && slot == 0 && lane_id() == 0) atomicAdd(p.err, (unsigned long long)__builtin_popcountll(bad));
-            for (; bad; bad &= bad - 1) {
-                T *dst = (T *)p.out + (b + __builtin_ctzll(bad)) * p.vec_size;
-                for (int64_t k = slot * kWave + lane_id(); k < p.vec_size; k += team * kWave) dst[k] = T(0);
+        return 0;
+    }
+    __device__ __forceinline__ uint64_t batched() const { return batched((3 * nrows + 3) / 4); }
+};
+
+// A window's rows in the team's LDS: where the stored rows start, their bytes,
+// their keys.
+constexpr int kWindowLdsWords = 5 * kWideWindow;
+
+// The part of a window that a team of two waves or more takes, in batches of
+// rows alike.  WHOLE (windows of kWideRows at most): all of it, in batches if all
+// its rows go together, else two waves per row.  One wave reads the rows'
+// metadata for the team.
+//
+// Batches of few rows cost as much as full ones, and a window's rows that go by
+// themselves wait for its batches: taken from two or four alike rows on, windows
+// of 16 evenly used mask rows lost up to 2.1 times a wave per row (2000 rows of
+// 1600 words 22 us against 46, now 16).  A batch's rows are unpacked four at a
+// time: with what the window keeps, eight put 22 to 28 registers in scratch
+// memory.  (Two at a time: 4096 x 2752 doubles from HBM 56 us, four 48.)
+template <typename T, typename IdxT, int LAYOUT, bool NT, bool WHOLE>
+__device__ __forceinline__ void fetch_wide_window(const FetchParams &p, int64_t b, int64_t e, int team, int slot,
+                                                  uint32_t *lds, uint32_t *rows)
+{
+    const WideBatch<T, LAYOUT, NT, 4> batch(p, team, slot, lds);
+    int64_t *const start = reinterpret_cast<int64_t *>(rows), *const stored = start + kWideWindow;
+    int *const keys = reinterpret_cast<int *>(stored + kWideWindow);
+    WideWindow<T> win;
+    batch.sync(); // the window before this one is done
+    if (slot == 0) {
+        win.template load<IdxT, LAYOUT>(p, b, e);
+        start[lane_id()] = win.m.word * (int64_t)sizeof(T);
+        stored[lane_id()] = win.m.len * (int64_t)sizeof(T);
+        keys[lane_id()] = win.key;
+    }
+    batch.sync();
+    win.nrows = (int)(e - b);
+    win.key = keys[lane_id()];
+    win.count();
+    if constexpr (WHOLE) {
+        if (!win.batched(win.nrows)) {
+            // Two waves a row.
+            const WideBatch<T, LAYOUT, NT, 1, true> one(p, 2, slot & 1, lds + (slot >> 1) * kWideStride);
+            for (int r0 = 0; r0 < win.nrows; r0 += team / 2) {
+                const int r = r0 + (slot >> 1);
+                const bool row = r < win.nrows; // the last pairs may have none
+                const int kind = row ? readlane(win.key, r) : -2;
+                WideRow part;
+                part.row = start[row ? r : 0];
+                part.stored = stored[row ? r : 0];
+                part.cursor = header_bytes(p.vec_size, (int)sizeof(T)) * 8;
+                part.out = 0;
+                if (p.host_rows && kind >= 0 && p.vec_size * (int64_t)sizeof(T) > 2048)
+                    touch_headers(p, (int)sizeof(T), part, 1, 1, 2, slot & 1);
+                if (row && kind == -2 && p.err && (slot & 1) == 0 && lane_id() == 0) atomicAdd(p.err, 1ull);
+                one.run(part, row ? 1 : 0, kind >= 0 ? 0xffu : 0u, kind == -1 ? 0xffu : 0u, kind < 0 ? 0 : kind, b + r);
             }
+            return;
         }
-        // (fewer than `least` of them go to a wave each, below)
-        uint64_t single = 0;
-        const int key = m.packed ? m.cl : -1; // raw rows need no mask row
-        while (left) {
-            const int kind = readlane(key, __builtin_ctzll(left)), cl = kind < 0 ? 0 : kind;
-            uint64_t alike = ballot(key == kind) & left;
-            left &= ~alike;
-            while (__builtin_popcountll(alike) >= least) {
-                // place k of the batch: the k-th of them; places past the last stand for the first
-                const int place = lane_id() & (kWideRows - 1);
-                int from = __builtin_ctzll(alike), n = 0;
+    }
+    for (uint64_t left = WHOLE ? win.ok : win.batched(); left;) {
+        const int head = __builtin_ctzll(left);
+        uint64_t alike = win.alike(head) & left;
+        left &= ~alike;
+        const int kind = readlane(win.key, head), cl = kind < 0 ? 0 : kind;
+        while (alike) {
+            // place k of the batch: the k-th of them; places past the last stand for the first
+            const int place = lane_id() & (kWideRows - 1);
+            int from = __builtin_ctzll(alike), n = 0;
 #pragma unroll
-                for (int k = 0; k < kWideRows; ++k) {
-                    if (!alike) break; // uniform
-                    const int at = __builtin_ctzll(alike);
-                    alike &= alike - 1;
-                    from = place == k ? at : from;
-                    ++n;
-                }
-                WideRow part = me;
-                part.row = (int64_t)shfl((uint64_t)me.row, from);
-                part.stored = (int64_t)shfl((uint64_t)me.stored, from);
-                part.out = (int64_t)from * (p.vec_size * (int64_t)sizeof(T));
-                const uint32_t part_pk = (uint32_t)ballot((pk >> from) & 1) & kLow;
-                batch.run(part, n, part_pk, kLow & ~part_pk, cl, b);
+            for (int k = 0; k < kWideRows; ++k) {
+                if (!alike) break; // uniform
+                const int at = __builtin_ctzll(alike);
+                alike &= alike - 1;
+                from = place == k ? at : from;
+                ++n;
             }
-            single |= alike;
-        }
-        for (int k = 0; single; ++k, single &= single - 1) {
-            const int at = __builtin_ctzll(single);
-            if (k % team == slot) fetch_large_row_from<T, LAYOUT>(p, b + at, readlane(s, at));
+            WideRow part;
+            part.row = start[from];
+            part.stored = stored[from];
+            part.cursor = header_bytes(p.vec_size, (int)sizeof(T)) * 8;
+            part.out = from;
+            constexpr uint32_t kLow = (1u << kWideRows) - 1;
+            if (p.host_rows && kind >= 0 && p.vec_size * (int64_t)sizeof(T) > 2048)
+                touch_headers(p, (int)sizeof(T), part, kLow, n, team, slot);
+            batch.run(part, n, kind < 0 ? 0u : kLow, kind < 0 ? kLow : 0u, cl, b);
         }
     }
 }

@@ -5,23 +5,45 @@
 
 namespace ibp {
 
-// Batches of rows_per_batch rows.  team > 1: a block is one team; team = 1:
-// each of a block's waves takes its own batches.
-template <typename T, typename IdxT, int LAYOUT, bool NT>
+// How a kernel of teams takes its rows: in batches of rows that follow each
+// other; with clusters in batches of one row, in whole windows, or the part of
+// a window that shares a mask row (fetch_wide_rest_kernel takes the others).
+enum : int { kBatches, kWholeWindows, kWindowParts };
+
+// Batches (windows) of rows_per_batch rows.  team > 1: a block is one team;
+// team = 1 (not with windows): each of a block's waves takes its own batches.
+template <typename T, typename IdxT, int LAYOUT, bool NT, int TAKE>
 __global__ __launch_bounds__(64 * kWideMaxTeam, 4) void fetch_wide_kernel(FetchParams p, int team, int rows_per_batch)
 {
     __shared__ uint32_t lds[kWideSolo][kWideLdsWords];
-    // With clusters: fewer rows of one mask row cost more in a batch than in a
-    // wave each, unless their window is so small that the team's other waves
-    // would have none (500 rows of 2752 words: 18 us against 51).
-    const int least = rows_per_batch <= 2 ? 1 : rows_per_batch <= 4 ? 2 : 4;
+    __shared__ __align__(8) uint32_t window[TAKE == kBatches ? 1 : kWindowLdsWords];
     const int wib = wave_in_block_id();
     const int64_t first = team > 1 ? (int64_t)blockIdx.x : global_wave_id();
     const int64_t step = team > 1 ? (int64_t)gridDim.x : (int64_t)gridDim.x * (blockDim.x / kWave);
     for (int64_t b = first * rows_per_batch; b < p.n; b += step * rows_per_batch) {
         const int64_t e = b + rows_per_batch < p.n ? b + rows_per_batch : p.n;
-        fetch_wide_batch<T, IdxT, LAYOUT, NT>(p, b, e, team, team > 1 ? wib : 0,
-                                              lds[team > 1 ? 0 : wib], least);
+        if constexpr (TAKE == kBatches)
+            fetch_wide_batch<T, IdxT, LAYOUT, NT>(p, b, e, team, team > 1 ? wib : 0, lds[team > 1 ? 0 : wib]);
+        else
+            fetch_wide_window<T, IdxT, LAYOUT, NT, TAKE == kWholeWindows>(p, b, e, team, wib, lds[0], window);
+    }
+}
+
+// A wave per row for the rows of windows of `rows` rows (a power of two) that
+// the teams leave.  (In the teams' kernel they had half the waves in flight, and
+// their code cost it scratch memory: 8192 rows of 800 doubles with 16 evenly used
+// mask rows 56 us, so 45; a wave per row for all of them 40.)
+template <typename T, typename IdxT, int LAYOUT>
+__global__ __launch_bounds__(256) void fetch_wide_rest_kernel(FetchParams p, int rows)
+{
+    const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / kWave);
+    for (int64_t i = global_wave_id(); i < p.n; i += nwaves) {
+        const int64_t b = i & ~(int64_t)(rows - 1);
+        const int r = (int)(i - b);
+        WideWindow<T> win;
+        win.template load<IdxT, LAYOUT>(p, b, b + rows < p.n ? b + rows : p.n);
+        if ((win.batched() >> r) & 1) continue; // uniform
+        fetch_large_row<T>(p, i, win.row(r));
     }
 }
 
@@ -30,10 +52,27 @@ namespace {
 template <typename T, typename IdxT, int LAYOUT>
 void launch_stores(const FetchParams &p, dim3 g, dim3 b, int team, int rows, hipStream_t s)
 {
-    if ((p.vec_size * (int64_t)sizeof(T)) % 128 == 0) // rows_fill_lines
-        hipLaunchKernelGGL((fetch_wide_kernel<T, IdxT, LAYOUT, true>), g, b, 0, s, p, team, rows);
-    else
-        hipLaunchKernelGGL((fetch_wide_kernel<T, IdxT, LAYOUT, false>), g, b, 0, s, p, team, rows);
+    auto take = [&](auto how) {
+        constexpr int TAKE = decltype(how)::value;
+        if ((p.vec_size * (int64_t)sizeof(T)) % 128 == 0) // rows_fill_lines
+            hipLaunchKernelGGL((fetch_wide_kernel<T, IdxT, LAYOUT, true, TAKE>), g, b, 0, s, p, team, rows);
+        else
+            hipLaunchKernelGGL((fetch_wide_kernel<T, IdxT, LAYOUT, false, TAKE>), g, b, 0, s, p, team, rows);
+    };
+    if constexpr ((LAYOUT & kLayoutClustered) != 0) {
+        if (rows > kWideRows) {
+            take(std::integral_constant<int, kWindowParts>());
+            const int64_t waves = p.n < (int64_t)1 << 20 ? p.n : (int64_t)1 << 20;
+            hipLaunchKernelGGL((fetch_wide_rest_kernel<T, IdxT, LAYOUT>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
+                               s, p, rows);
+            return;
+        }
+        if (rows > 1) {
+            take(std::integral_constant<int, kWholeWindows>());
+            return;
+        }
+    }
+    take(std::integral_constant<int, kBatches>());
 }
 
 template <typename T, typename IdxT>
@@ -53,11 +92,11 @@ void launch_layout(const FetchParams &p, int layout, dim3 g, dim3 b, int team, i
 // columns on always (200 rows of 600 words: a wave per row 8.8 us, teams 5.9;
 // of 400: 7.0 and 8.1 at 1000 rows), below from 8 MB of rows on (60,000 rows of
 // 118 words 28 and 22 us, 8000 6.8 and 9.5; 12,000 rows of 256 words 12.8 and
-// 9.6, 4000 6.6 and 8.5).  A mask row per cluster: rows of 6 KB and more
-// (8192 rows of 2500 doubles with 16 of them: 135 and 85, 249 and 96, 120 and
-// 82 us on weights, node features and embeddings, whose rows mostly share few
-// mask rows; 107 and 140 where the sixteen are evenly used; of 500 doubles 34
-// and 38).
+// 9.6, 4000 6.6 and 8.5).  A mask row per cluster: rows of 6 KB and more.  All
+// rows of one mask row (weights, node features, embeddings mostly): 2000, 4096
+// and 30,000 rows of 800 doubles 16, 23 and 130 us by a wave per row and 13, 15
+// and 87 by teams, of 2752 doubles (16,000) 51, 75 and 240 and 24, 33 and 135.
+// Sixteen evenly used: 16, 24, 130 and 15, 25, 140; 52, 76, 239 and 38, 76, 244.
 bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes)
 {
     if (p.vec_size <= kWave || elem_bytes < 4) return false;
@@ -76,11 +115,18 @@ int fetch_wide_launch(const FetchParams &p, int layout, int elem_bytes, int inde
     // rows of eight chunks: teams of 2, 4, 8 take 32.9, 29.8, 34.4 us; 4096
     // rows of 43 chunks: teams of 4 and 8 take 53 and 45 us).
     const int most = nchunks <= 1 ? 1 : nchunks <= 2 ? 2 : nchunks <= 4 ? 4 : kWideMaxTeam;
-    const int most_rows = (layout & kLayoutClustered) ? kWideWindow : kWideRows;
-    int rows = 1;
-    while (rows < most_rows && (p.n + rows - 1) / rows * most > (int64_t)dev.num_cus * 16) rows *= 2;
-    int team = most < 2 ? most : 2;
-    while (team < most && (p.n + rows - 1) / rows * team < (int64_t)dev.num_cus * 32) team *= 2;
+    const bool clustered = (layout & kLayoutClustered) != 0;
+    const int most_rows = clustered ? kWideWindow : kWideRows;
+    int rows = 1, team = most < 2 ? most : 2;
+    // With clusters and four waves or more for a row, rows by themselves: which
+    // mask rows they use does not matter then (1000 rows of 800 and 2752
+    // doubles: 10 and 19 us; windows of two rows of other mask rows 14 and 31).
+    if (clustered && p.n * 4 <= (int64_t)dev.num_cus * 16) {
+        while (team < most && p.n * team * 2 <= (int64_t)dev.num_cus * 16) team *= 2;
+    } else {
+        while (rows < most_rows && (p.n + rows - 1) / rows * most > (int64_t)dev.num_cus * 16) rows *= 2;
+        while (team < most && (p.n + rows - 1) / rows * team < (int64_t)dev.num_cus * 32) team *= 2;
+    }
     const int waves = team > 1 ? team : kWideSolo;
     int64_t grid = ((p.n + rows - 1) / rows * team + waves - 1) / waves;
     if (grid > (int64_t)1 << 20) grid = (int64_t)1 << 20;
