@@ -76,9 +76,10 @@ int ibp_preprocess(int elem_bytes, const void *data, int64_t num_vecs, int64_t v
  * touched); seed < 0 continues the process-wide rand() state like the
  * reference.  threshold is accepted and ignored, as in the reference.
  * Synchronises the stream before returning.  The *_ws form takes device memory
- * (256-byte aligned) of ibp_preprocess_kmeans_workspace_size() bytes (less runs
- * too, slower, down to what the call needs without its copy of the rows), or
- * NULL to let the library allocate (stream-ordered). */
+ * (256-byte aligned) of ibp_preprocess_kmeans_workspace_size() bytes, or NULL to
+ * let the library allocate (stream-ordered).  With up to 16 clusters these bytes
+ * hold a copy of the rows, up to 2 GiB of them; where the call needs less
+ * without it, less memory runs too, slower (the error names the least). */
 int ibp_preprocess_kmeans(int elem_bytes, const void *data, int64_t num_vecs, int64_t vec_size,
                           int num_clusters, float threshold, int64_t seed, void *masks,
                           void *bitvals, int32_t *clusters, void *stream);

@@ -895,19 +895,21 @@ int kmeans_typed(const void *data_v, int64_t N, int64_t V, int K, int64_t seed, 
     }
 
     // The caller's workspace, or an allocation; without the bit planes where
-    // that is too small for them or memory is short.
+    // that is too small for them or memory is short, and they are what takes
+    // the memory (few wide rows need more without them, for partial counts).
     KmPlan pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, true);
+    const KmPlan less = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
     unsigned char *ws = (unsigned char *)workspace;
     hipError_t e = hipSuccess;
     if (workspace) {
-        if (workspace_bytes < pl.total) pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
+        if (workspace_bytes < pl.total && less.total < pl.total) pl = less;
         if (workspace_bytes < pl.total)
             return set_error(IBP_ERR_INVALID, "workspace too small (%zu < %zu bytes)", workspace_bytes, pl.total);
     } else {
         e = hipMallocAsync((void **)&ws, pl.total, s);
-        if (e != hipSuccess && pl.planes) {
+        if (e != hipSuccess && less.total < pl.total) {
             (void)hipGetLastError();
-            pl = plan_kmeans(dev, (int)sizeof(T), N, V, K, false);
+            pl = less;
             e = hipMallocAsync((void **)&ws, pl.total, s);
         }
         if (e != hipSuccess)
