@@ -28,7 +28,8 @@ int fetch_launch(const FetchParams &p, int elem_bytes, int index_bytes, int impl
                  int nthreads, hipStream_t stream, int layout, bool host_resident)
 {
     const DeviceInfo &dev = device_info();
-    // Blocks are at most 256 threads (four waves); larger requests are capped.
+    // Blocks are at most 256 threads (four waves; teams of waves: 512); larger
+    // requests are capped.
     const int block = (nthreads > 0 && nthreads <= 256) ? nthreads : 256;
     int rows = g_rows_in_flight.load();
 #ifndef IBP_NO_SMALL_CALL_ROWS
@@ -40,7 +41,8 @@ int fetch_launch(const FetchParams &p, int elem_bytes, int index_bytes, int impl
         while (rows > 2 && (p.n + rows - 1) / rows < want) rows /= 2;
     }
 #endif
-    const bool wide = impl != 2 && impl != 3 && impl != 4 && fetch_wide_pays(p, layout, elem_bytes);
+    const bool wide = impl != 2 && impl != 3 && impl != 4 && fetch_wide_pays(p, layout, elem_bytes, nthreads);
+    const WideShape shape = wide ? fetch_wide_shape(p, layout, elem_bytes, nblks, nthreads) : WideShape{};
     int64_t waves_needed = p.vec_size <= kWave ? (p.n + rows - 1) / rows : p.n;
     int64_t grid = nblks > 0 ? nblks : (waves_needed * kWave + block - 1) / block;
     int64_t cap = (int64_t)dev.num_cus * g_blocks_per_cu.load();
@@ -60,9 +62,10 @@ int fetch_launch(const FetchParams &p, int elem_bytes, int index_bytes, int impl
         dprintf("[ibp] decompress_fetch: %s, impl %d, %s rows, V=%lld, w=%d, n=%lld, grid %lld x %d, rows in flight %d, "
                 "first read %d words, comp_len %d\n",
                 kind, impl, host_resident ? "host (PCIe)" : "device", (long long)p.vec_size, elem_bytes,
-                (long long)p.n, (long long)grid, block, p.vec_size <= kWave ? rows : 1, p.first_words, comp_len);
+                (long long)p.n, (long long)(wide ? shape.grid : grid), wide ? shape.block : block,
+                wide ? shape.rows : p.vec_size <= kWave ? rows : 1, p.first_words, comp_len);
     }
-    if (wide) return fetch_wide_launch(p, layout, elem_bytes, index_bytes, nblks, stream);
+    if (wide) return fetch_wide_launch(p, layout, elem_bytes, index_bytes, nblks, shape, stream);
     switch (elem_bytes) {
     case 1: return fetch_launch_width<uint8_t>(p, layout, index_bytes, impl, comp_len, rows, (int)grid, block, stream);
     case 2: return fetch_launch_width<uint16_t>(p, layout, index_bytes, impl, comp_len, rows, (int)grid, block, stream);

@@ -736,10 +736,18 @@ __device__ __forceinline__ void fetch_wide_window(const FetchParams &p, int64_t 
 }
 
 // Whether teams of waves are the faster way (else a wave per row).
-bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes);
+bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes, int nthreads);
 // The plain fetch's launch for rows of more than 64 elements of 4 or 8 bytes
-// (ibp_fetch_wide.hip); nblks <= 0: a grid for the rows.
+// (ibp_fetch_wide.hip).  nblks <= 0: a grid for the rows; nthreads > 0: threads
+// of a block, at most.
+struct WideShape {
+    int64_t grid;
+    int block; // threads
+    int team;  // waves
+    int rows;  // of a batch, or of a window
+};
+WideShape fetch_wide_shape(const FetchParams &p, int layout, int elem_bytes, int nblks, int nthreads);
 int fetch_wide_launch(const FetchParams &p, int layout, int elem_bytes, int index_bytes, int nblks,
-                      hipStream_t stream);
+                      const WideShape &shape, hipStream_t stream);
 
 } // namespace ibp

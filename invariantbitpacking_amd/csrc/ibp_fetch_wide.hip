@@ -50,8 +50,10 @@ __global__ __launch_bounds__(256) void fetch_wide_rest_kernel(FetchParams p, int
 namespace {
 
 template <typename T, typename IdxT, int LAYOUT>
-void launch_stores(const FetchParams &p, dim3 g, dim3 b, int team, int rows, hipStream_t s)
+void launch_stores(const FetchParams &p, const WideShape &w, int nblks, hipStream_t s)
 {
+    const dim3 g((unsigned)w.grid), b((unsigned)w.block);
+    const int team = w.team, rows = w.rows;
     auto take = [&](auto how) {
         constexpr int TAKE = decltype(how)::value;
         if ((p.vec_size * (int64_t)sizeof(T)) % 128 == 0) // rows_fill_lines
@@ -62,8 +64,10 @@ void launch_stores(const FetchParams &p, dim3 g, dim3 b, int team, int rows, hip
     if constexpr ((LAYOUT & kLayoutClustered) != 0) {
         if (rows > kWideRows) {
             take(std::integral_constant<int, kWindowParts>());
+            const int block = w.block < 256 ? w.block : 256;
             const int64_t waves = p.n < (int64_t)1 << 20 ? p.n : (int64_t)1 << 20;
-            hipLaunchKernelGGL((fetch_wide_rest_kernel<T, IdxT, LAYOUT>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
+            const int64_t blocks = nblks > 0 ? nblks : (waves * kWave + block - 1) / block;
+            hipLaunchKernelGGL((fetch_wide_rest_kernel<T, IdxT, LAYOUT>), dim3((unsigned)blocks), dim3((unsigned)block), 0,
                                s, p, rows);
             return;
         }
@@ -76,13 +80,13 @@ void launch_stores(const FetchParams &p, dim3 g, dim3 b, int team, int rows, hip
 }
 
 template <typename T, typename IdxT>
-void launch_layout(const FetchParams &p, int layout, dim3 g, dim3 b, int team, int rows, hipStream_t s)
+void launch_layout(const FetchParams &p, int layout, const WideShape &w, int nblks, hipStream_t s)
 {
     switch (layout) {
-    case kLayoutSlots: launch_stores<T, IdxT, kLayoutSlots>(p, g, b, team, rows, s); break;
-    case kLayoutCondensed: launch_stores<T, IdxT, kLayoutCondensed>(p, g, b, team, rows, s); break;
-    case kLayoutClustered: launch_stores<T, IdxT, kLayoutClustered>(p, g, b, team, rows, s); break;
-    default: launch_stores<T, IdxT, kLayoutCondensed | kLayoutClustered>(p, g, b, team, rows, s); break;
+    case kLayoutSlots: launch_stores<T, IdxT, kLayoutSlots>(p, w, nblks, s); break;
+    case kLayoutCondensed: launch_stores<T, IdxT, kLayoutCondensed>(p, w, nblks, s); break;
+    case kLayoutClustered: launch_stores<T, IdxT, kLayoutClustered>(p, w, nblks, s); break;
+    default: launch_stores<T, IdxT, kLayoutCondensed | kLayoutClustered>(p, w, nblks, s); break;
     }
 }
 
@@ -97,15 +101,16 @@ void launch_layout(const FetchParams &p, int layout, dim3 g, dim3 b, int team, i
 // and 30,000 rows of 800 doubles 16, 23 and 130 us by a wave per row and 13, 15
 // and 87 by teams, of 2752 doubles (16,000) 51, 75 and 240 and 24, 33 and 135.
 // Sixteen evenly used: 16, 24, 130 and 15, 25, 140; 52, 76, 239 and 38, 76, 244.
-bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes)
+// (With blocks of one wave, by nthreads, a window has no team.)
+bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes, int nthreads)
 {
     if (p.vec_size <= kWave || elem_bytes < 4) return false;
     const int64_t row_bytes = p.vec_size * elem_bytes;
-    if (layout & kLayoutClustered) return row_bytes >= 6144;
+    if (layout & kLayoutClustered) return row_bytes >= 6144 && (nthreads <= 0 || nthreads >= 2 * kWave);
     return p.vec_size >= 512 || p.n >= ((int64_t)8 << 20) / row_bytes;
 }
 
-int fetch_wide_launch(const FetchParams &p, int layout, int elem_bytes, int index_bytes, int nblks, hipStream_t stream)
+WideShape fetch_wide_shape(const FetchParams &p, int layout, int elem_bytes, int nblks, int nthreads)
 {
     const DeviceInfo &dev = device_info();
     const int64_t nchunks = (p.vec_size * elem_bytes + 511) / 512;
@@ -114,32 +119,40 @@ int fetch_wide_launch(const FetchParams &p, int layout, int elem_bytes, int inde
     // the chip twice that, since a smaller team shares fewer barriers (20,000
     // rows of eight chunks: teams of 2, 4, 8 take 32.9, 29.8, 34.4 us; 4096
     // rows of 43 chunks: teams of 4 and 8 take 53 and 45 us).
-    const int most = nchunks <= 1 ? 1 : nchunks <= 2 ? 2 : nchunks <= 4 ? 4 : kWideMaxTeam;
+    int most = nchunks <= 1 ? 1 : nchunks <= 2 ? 2 : nchunks <= 4 ? 4 : kWideMaxTeam;
+    while (nthreads > 0 && most > 1 && most * kWave > nthreads) most /= 2;
     const bool clustered = (layout & kLayoutClustered) != 0;
     const int most_rows = clustered ? kWideWindow : kWideRows;
-    int rows = 1, team = most < 2 ? most : 2;
+    WideShape w{0, 0, most < 2 ? most : 2, 1};
     // With clusters and four waves or more for a row, rows by themselves: which
     // mask rows they use does not matter then (1000 rows of 800 and 2752
     // doubles: 10 and 19 us; windows of two rows of other mask rows 14 and 31).
     if (clustered && p.n * 4 <= (int64_t)dev.num_cus * 16) {
-        while (team < most && p.n * team * 2 <= (int64_t)dev.num_cus * 16) team *= 2;
+        while (w.team < most && p.n * w.team * 2 <= (int64_t)dev.num_cus * 16) w.team *= 2;
     } else {
-        while (rows < most_rows && (p.n + rows - 1) / rows * most > (int64_t)dev.num_cus * 16) rows *= 2;
-        while (team < most && (p.n + rows - 1) / rows * team < (int64_t)dev.num_cus * 32) team *= 2;
+        while (w.rows < most_rows && (p.n + w.rows - 1) / w.rows * most > (int64_t)dev.num_cus * 16) w.rows *= 2;
+        while (w.team < most && (p.n + w.rows - 1) / w.rows * w.team < (int64_t)dev.num_cus * 32) w.team *= 2;
     }
-    const int waves = team > 1 ? team : kWideSolo;
-    int64_t grid = ((p.n + rows - 1) / rows * team + waves - 1) / waves;
-    if (grid > (int64_t)1 << 20) grid = (int64_t)1 << 20;
-    if (nblks > 0) grid = nblks;
-    if (grid < 1) grid = 1;
-    const dim3 g((unsigned)grid), b((unsigned)(waves * kWave));
+    int waves = w.team > 1 ? w.team : kWideSolo;
+    if (nthreads > 0 && waves * kWave > nthreads) waves = nthreads / kWave;
+    w.block = waves * kWave;
+    w.grid = ((p.n + w.rows - 1) / w.rows * w.team + waves - 1) / waves;
+    if (w.grid > (int64_t)1 << 20) w.grid = (int64_t)1 << 20;
+    if (nblks > 0) w.grid = nblks;
+    if (w.grid < 1) w.grid = 1;
+    return w;
+}
+
+int fetch_wide_launch(const FetchParams &p, int layout, int elem_bytes, int index_bytes, int nblks, const WideShape &w,
+                      hipStream_t stream)
+{
     const bool i32 = p.index != nullptr && index_bytes == 4;
     if (elem_bytes == 8) {
-        if (i32) launch_layout<uint64_t, int32_t>(p, layout, g, b, team, rows, stream);
-        else launch_layout<uint64_t, int64_t>(p, layout, g, b, team, rows, stream);
+        if (i32) launch_layout<uint64_t, int32_t>(p, layout, w, nblks, stream);
+        else launch_layout<uint64_t, int64_t>(p, layout, w, nblks, stream);
     } else {
-        if (i32) launch_layout<uint32_t, int32_t>(p, layout, g, b, team, rows, stream);
-        else launch_layout<uint32_t, int64_t>(p, layout, g, b, team, rows, stream);
+        if (i32) launch_layout<uint32_t, int32_t>(p, layout, w, nblks, stream);
+        else launch_layout<uint32_t, int64_t>(p, layout, w, nblks, stream);
     }
     IBP_LAUNCH_CHECK();
     return IBP_OK;
