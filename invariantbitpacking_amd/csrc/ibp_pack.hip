@@ -1580,9 +1580,11 @@ int pack_width(const PackParams &p, int index_bytes, hipStream_t s)
     // against 45 to 288 here, the copy of the table included), narrower ones
     // from 32768 rows on (60,000 rows of 65 words 59 against 81, 16,000 rows 40
     // against 34).  Rows in host memory stay with a wave each (52 against 46
-    // GB/s over PCIe, 4096 rows of 1024 and 2752 doubles).
+    // GB/s over PCIe, 4096 rows of 1024 and 2752 doubles), and so do packs
+    // whose bitmask is there: the teams set its bits with an atomic OR, which
+    // PCIe does not have.
     if (sizeof(T) >= 4 && p.V > kWave && p.V * (int64_t)sizeof(T) <= kPackWideMaxBytes &&
-        (p.V >= 512 || p.n >= 32768) && !pointer_is_host(p.in))
+        (p.V >= 512 || p.n >= 32768) && !pointer_is_host(p.in) && !(p.bitmask && pointer_is_host(p.bitmask)))
         return pack_wide_launch(p, (int)sizeof(T), index_bytes, s);
     const bool i32 = p.index && index_bytes == 4;
     if (p.offsets)
