@@ -1578,13 +1578,20 @@ int pack_width(const PackParams &p, int index_bytes, hipStream_t s)
     // Teams of waves per row (ibp_pack_wide.hip): rows of 512 columns and more
     // whatever their number (500 to 60,000 rows of 600 words: 28 to 192 us,
     // against 45 to 288 here, the copy of the table included), narrower ones
-    // from 32768 rows on (60,000 rows of 65 words 59 against 81, 16,000 rows 40
-    // against 34).  Rows in host memory stay with a wave each (52 against 46
-    // GB/s over PCIe, 4096 rows of 1024 and 2752 doubles), and so do packs
-    // whose bitmask is there: the teams set its bits with an atomic OR, which
-    // PCIe does not have.
-    if (sizeof(T) >= 4 && p.V > kWave && p.V * (int64_t)sizeof(T) <= kPackWideMaxBytes &&
-        (p.V >= 512 || p.n >= 32768) && !pointer_is_host(p.in) && !(p.bitmask && pointer_is_host(p.bitmask)))
+    // from 32768 rows on (40,000 rows of 200 words 68 against 77), of less than
+    // 800 bytes from 49152 (40,000 rows of 65 words 56 against 52, 60,000 62 and
+    // 69).  But slots of less than 3 KiB that fill half the CUs' blocks of 32
+    // rows or more, and all of them at most once, stay here (8000 rows of 512,
+    // 600 and 700 words that pack to 40%: 46, 52 and 52 us by teams, here 39, 45
+    // and 47).  Rows in host memory stay with a wave each (52 against 46 GB/s
+    // over PCIe, 4096 rows of 1024 and 2752 doubles), and so do packs whose
+    // bitmask is there: the teams set its bits with an atomic OR, which PCIe
+    // does not have.
+    const int64_t row_bytes = p.V * (int64_t)sizeof(T), cus = device_info().num_cus;
+    const bool one_round = !p.offsets && row_bytes < 3072 && p.n > cus * 16 && p.n <= cus * 32;
+    if (sizeof(T) >= 4 && p.V > kWave && row_bytes <= kPackWideMaxBytes &&
+        (p.V >= 512 ? !one_round : p.n >= (row_bytes >= 800 ? 32768 : 49152)) && !pointer_is_host(p.in) &&
+        !(p.bitmask && pointer_is_host(p.bitmask)))
         return pack_wide_launch(p, (int)sizeof(T), index_bytes, s);
     const bool i32 = p.index && index_bytes == 4;
     if (p.offsets)

@@ -284,7 +284,12 @@ int pack_wide_launch(const PackParams &p, int elem_bytes, int index_bytes, hipSt
     const int waves = team > 1 ? team : kSoloWaves;
     const size_t lds = (size_t)((row_bytes + 15) / 16 * 16 + kWave * 4) * (team > 1 ? 1 : waves);
     int64_t grid = (p.n * team + waves - 1) / waves;
-    const int64_t cap = (int64_t)dev.num_cus * 128 / waves;
+    // A small team's block takes more rows while they are few, since its start
+    // costs more than a row (8000 and 16,000 rows of 600 words: 32 waves' blocks
+    // per CU 51.7 and 70.0 us, 128 waves' 55.0 and 72.9; 48,000 rows 145.6 and
+    // 141.2; 8000 rows of 1200 doubles 113 and 103).
+    const bool few = team <= 4 && p.n * team <= (int64_t)dev.num_cus * 256;
+    const int64_t cap = (int64_t)dev.num_cus * (few ? 32 : 128) / waves;
     if (grid > cap) grid = cap;
     if (p.bitmask) {
         const int64_t words = (p.n + 31) / 32;
@@ -292,6 +297,8 @@ int pack_wide_launch(const PackParams &p, int elem_bytes, int index_bytes, hipSt
                            stream, p.bitmask, words);
         IBP_LAUNCH_CHECK();
     }
+    dprintf("[ibp] compress: team of %d waves per row, V=%lld, w=%d, n=%lld, grid %lld x %d\n", team, (long long)p.V,
+            elem_bytes, (long long)p.n, (long long)grid, waves * kWave);
     const dim3 g((unsigned)grid), b((unsigned)(waves * kWave));
     const bool i32 = p.index && index_bytes == 4, condensed = p.offsets != nullptr;
     if (elem_bytes == 8) launch<uint64_t>(p, i32, condensed, cpw, g, b, lds, team, stream);
