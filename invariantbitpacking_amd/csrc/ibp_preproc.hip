@@ -215,7 +215,8 @@ __global__ __launch_bounds__(1024) void masks_kernel(const int32_t *part, int64_
             masks[t * V + j] = m[t];
             bitvals[t * V + j] = v;
         }
-        if (lane == 0) atomicAdd(&total->flagged[blockIdx.x % Sums::kCopies].t[t], (unsigned long long)__builtin_popcountll(all));
+        if (recs && lane == 0) // only the slices' scores start from them
+            atomicAdd(&total->flagged[blockIdx.x % Sums::kCopies].t[t], (unsigned long long)__builtin_popcountll(all));
     }
     if constexpr (sizeof(T) >= 4) {
         if (recs && lane < COLS && j < V) {
@@ -669,9 +670,14 @@ int preprocess_typed(const void *data, int64_t N, int64_t V, const Thresholds &t
     }
     IBP_LAUNCH_CHECK();
     // Rows of 4- or 8-byte elements and at least 16 bytes: lane <-> row, from
-    // the score units; narrower ones: lane <-> column.
+    // the score units; narrower ones: lane <-> column.  So too, with one
+    // threshold, tables of very wide rows that are few: a wave per row, where a
+    // tile's waves walk its slices in turn (100 x 4096 doubles: 59 us per call
+    // and 76, 400 x 8000 109 and 133, 1000 x 2752 76 and 62; 20 x 20,000 floats
+    // 138 and 150, 400 162 and 160).
+    const bool few_wide = th.count == 1 && V > 2048 && N * (sizeof(T) == 8 ? 6 : 256) < V;
     const bool slices = sizeof(T) >= 4 && N > 0 && V * (int64_t)sizeof(T) >= 16 && V <= (int64_t)1 << 20 &&
-                        (uintptr_t)data % 4 == 0 && (th.count == 1 || th.count == kSweep);
+                        (uintptr_t)data % 4 == 0 && (th.count == 1 || th.count == kSweep) && !few_wide;
     const int64_t rgrid = (ncnt + kWave - 1) / kWave;
     hipLaunchKernelGGL((masks_kernel<T>), dim3((unsigned)rgrid), dim3(kWave * kReduceWaves), 0, stream,
                        (const int32_t *)part, row_blocks, N, V, th, masks, bitvals, slices ? recs : nullptr, sums);
