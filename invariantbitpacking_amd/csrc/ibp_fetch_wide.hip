@@ -119,7 +119,11 @@ WideShape fetch_wide_shape(const FetchParams &p, int layout, int elem_bytes, int
     // the chip twice that, since a smaller team shares fewer barriers (20,000
     // rows of eight chunks: teams of 2, 4, 8 take 32.9, 29.8, 34.4 us; 4096
     // rows of 43 chunks: teams of 4 and 8 take 53 and 45 us).
+    // Of five to seven chunks teams of eight leave waves idle, which many rows
+    // feel (16,000 rows of 600 words 36 us, by teams of four 26; 2000 rows 9.2
+    // and 10.3).
     int most = nchunks <= 1 ? 1 : nchunks <= 2 ? 2 : nchunks <= 4 ? 4 : kWideMaxTeam;
+    if (nchunks < most && p.n >= (int64_t)dev.num_cus * 24) most = 4;
     while (nthreads > 0 && most > 1 && most * kWave > nthreads) most /= 2;
     const bool clustered = (layout & kLayoutClustered) != 0;
     const int most_rows = clustered ? kWideWindow : kWideRows;
