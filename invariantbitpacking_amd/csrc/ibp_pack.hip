@@ -1305,9 +1305,12 @@ int size_typed(const void *data, int64_t num_vecs, int64_t V, const void *mask, 
         // x 20 doubles: 56 us, slices 63; 448-byte rows, five tiles: 36 and
         // 24).  Others in slices, but for rows of more than 1 KB that are too
         // few to give every CU half a tile (4000 x 1100 doubles: slices 14.7
-        // us, a wave per row 9.0; 8000: 16.7 and 17.5).
+        // us, a wave per row 9.0; 8000: 16.7 and 17.5).  Rows of more than 288
+        // bytes in host memory: a wave per row reads each end to end, which
+        // PCIe carries faster than the slices of many rows (9000 x 2752 doubles
+        // 3.46 ms and 4.54, 200,000 x 64 1.78 and 2.37, x 65 floats equal).
         const int64_t row_bytes = V * (int64_t)sizeof(T);
-        const bool whole = !index && !clusters && n == num_vecs && n > 0;
+        const bool whole = !index && !clusters && n == num_vecs && n > 0 && !(row_bytes > 288 && pointer_is_host(data));
         if (whole && tile_rows_ok(row_bytes) && row_bytes * kWave * 6 <= 160 * 1024 && ((uintptr_t)data % 16) == 0) {
             const size_t lds = (size_t)kWave * V * sizeof(T);
             int64_t per_cu = (int64_t)(160 * 1024) / (int64_t)lds;

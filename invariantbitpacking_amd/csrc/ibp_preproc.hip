@@ -676,8 +676,13 @@ int preprocess_typed(const void *data, int64_t N, int64_t V, const Thresholds &t
     // and 76, 400 x 8000 109 and 133, 1000 x 2752 76 and 62; 20 x 20,000 floats
     // 138 and 150, 400 162 and 160).
     const bool few_wide = th.count == 1 && V > 2048 && N * (sizeof(T) == 8 ? 6 : 256) < V;
+    // And rows of 320 bytes and more in host memory, which a wave reads end to
+    // end: PCIe carries slices of many rows 15% slower (200,000 x 50 doubles 3.20
+    // ms per call, so 2.88; 5000 x 2752 4.44 and 3.85; 200,000 x 75 floats,
+    // sweep, 2.40 and 2.49).
+    const bool over_pcie = V * (int64_t)sizeof(T) >= 320 && N > 0 && pointer_is_host(data);
     const bool slices = sizeof(T) >= 4 && N > 0 && V * (int64_t)sizeof(T) >= 16 && V <= (int64_t)1 << 20 &&
-                        (uintptr_t)data % 4 == 0 && (th.count == 1 || th.count == kSweep) && !few_wide;
+                        (uintptr_t)data % 4 == 0 && (th.count == 1 || th.count == kSweep) && !few_wide && !over_pcie;
     const int64_t rgrid = (ncnt + kWave - 1) / kWave;
     hipLaunchKernelGGL((masks_kernel<T>), dim3((unsigned)rgrid), dim3(kWave * kReduceWaves), 0, stream,
                        (const int32_t *)part, row_blocks, N, V, th, masks, bitvals, slices ? recs : nullptr, sums);
