@@ -217,7 +217,6 @@ int64_t fill_tasks(const ibp_fetch_task *tasks, int n, const BatchConfig &cfg, i
         d.p.n = t.n;
         const bool host = t.comp_loc == IBP_LOC_HOST || (t.comp_loc == IBP_LOC_AUTO && pointer_is_host(t.comp));
         d.p.first_words = first_words_for(t.vec_size, t.elem_bytes, t.comp_len, host);
-        d.p.host_rows = host ? 1 : 0;
         d.p.err = (t.index || t.offsets) ? index_error_counter() : nullptr;
         d.p.offsets = t.offsets;
         d.p.stream_bytes = t.stream_bytes;

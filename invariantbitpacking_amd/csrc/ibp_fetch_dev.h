@@ -46,7 +46,7 @@ struct FetchParams {
     int64_t vec_size = 0;
     int64_t n = 0;
     int32_t first_words = 0; // words read before the header is known (small rows)
-    int32_t host_rows = 0;   // comp is host memory, read over PCIe
+    int32_t host_rows = 0;   // comp is host memory, read over PCIe (teams of waves)
     unsigned long long *err = nullptr;
     const int64_t *offsets = nullptr;  // condensed layout
     const int32_t *clusters = nullptr; // clustered layout

@@ -182,7 +182,7 @@ __device__ __forceinline__ void size_score_chunk(const uint4 &v, const T (&m)[16
 {
 #pragma unroll
     for (int e = 0; e < (int)(16 / sizeof(T)); ++e)
-        lost = lost_step<true>(xor_ordered(chunk_elem<T>(v, e), b[e]), m[e], (uint32_t)popc(m[e]), lost);
+        lost = lost_step(xor_ordered(chunk_elem<T>(v, e), b[e]), m[e], (uint32_t)popc(m[e]), lost);
 }
 
 template <typename T>
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kWave) void size_tile_kernel(const T *__restrict__ 
     const int sw = tile_swz(lane, swz); // chunk c of this lane's row sits at c ^ sw
     unsigned long long acc = 0;
     for (int64_t tl = blockIdx.x; tl < ntiles; tl += gridDim.x) {
-        copy_tile<T, 1>(data, num_vecs, V, C, tl, 0, lane, tile, swz);
+        copy_tile<T>(data, num_vecs, V, C, tl, lane, tile, swz);
         __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): the tile has landed
         __builtin_amdgcn_wave_barrier();
         uint32_t lost = 0;
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void size_slices_ker
 #pragma unroll
         for (int e = 0; e < EPC; ++e) {
             const T m = e < shared ? T(0) : u.m[e];
-            lost = lost_step<true>(xor_ordered(chunk_elem<T>(v, e), u.b[e]), m, (uint32_t)popc(m), lost);
+            lost = lost_step(xor_ordered(chunk_elem<T>(v, e), u.b[e]), m, (uint32_t)popc(m), lost);
         }
     };
     int tile = SPLIT == 1 ? (int)blockIdx.x * WAVES + wv : (int)blockIdx.x;
@@ -1014,7 +1014,7 @@ __device__ __forceinline__ void pack_tile_body(const PackTileParams &p, T *__res
     const int q64 = kWave / C, r64 = kWave % C;
     const int wr0 = lane / C, wc0 = lane - (lane / C) * C;
     for (int64_t tl = blockIdx.x; tl < ntiles; tl += gridDim.x) {
-        copy_tile<T, 1>(data, p.num_vecs, V, C, tl, 0, lane, tile, swz);
+        copy_tile<T>(data, p.num_vecs, V, C, tl, lane, tile, swz);
         __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): the tile has landed
         __builtin_amdgcn_wave_barrier();
         const int64_t r = tl * kWave + lane;
@@ -1116,7 +1116,7 @@ __device__ __forceinline__ void pack_tile_condensed_body(const PackTileParams &p
     const int swe = sw * EPC;
     int bad = 0;
     for (int64_t tl = blockIdx.x; tl < ntiles; tl += gridDim.x) {
-        copy_tile<T, 1>(data, p.num_vecs, V, C, tl, 0, lane, tile, swz);
+        copy_tile<T>(data, p.num_vecs, V, C, tl, lane, tile, swz);
         const int64_t r = tl * kWave + lane;
         const bool in = r < p.num_vecs;
         const int64_t lo = in && r > 0 ? p.offsets[r - 1] : 0;

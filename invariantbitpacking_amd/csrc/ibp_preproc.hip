@@ -446,13 +446,13 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
             if constexpr (sizeof(T) == 8) {
                 const T d = xor_ordered((T)x0 | ((T)((uint64_t)x1 << 32)), x.b[0]);
 #pragma unroll
-                for (int t = 0; t < NA; ++t) lost[t] = lost_step<true>(d, x.m[0][t], x.p[0][t], lost[t]);
+                for (int t = 0; t < NA; ++t) lost[t] = lost_step(d, x.m[0][t], x.p[0][t], lost[t]);
             } else {
                 const T d0 = xor_ordered((T)x0, x.b[0]), d1 = xor_ordered((T)x1, x.b[R::EPU - 1]);
 #pragma unroll
                 for (int t = 0; t < NA; ++t) {
-                    lost[t] = lost_step<true>(d0, x.m[0][t], x.p[0][t], lost[t]);
-                    lost[t] = lost_step<true>(d1, x.m[R::EPU - 1][t], x.p[R::EPU - 1][t], lost[t]);
+                    lost[t] = lost_step(d0, x.m[0][t], x.p[0][t], lost[t]);
+                    lost[t] = lost_step(d1, x.m[R::EPU - 1][t], x.p[R::EPU - 1][t], lost[t]);
                 }
             }
         };

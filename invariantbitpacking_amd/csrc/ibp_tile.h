@@ -27,13 +27,13 @@ __host__ __device__ constexpr bool tile_rows_ok(int64_t row_bytes)
 // The XOR applied to the chunk index of tile row r (0 without the swizzle).
 __device__ __forceinline__ int tile_swz(int r, bool swz) { return swz ? (r & 7) : 0; }
 
-// The copy of tile tl (rows tl*64 ...) into `buf` by wave `wib` of WPT: 16-byte
-// chunks wib, wib + WPT, ... of the tile, each instruction 1 KB of consecutive
-// bytes straight to LDS (global_load_lds_dwordx4: no registers, tracked by
-// vmcnt).  C = row bytes / 16; swz: the placement above (then C % 8 == 0, and
-// the lane of LDS chunk g loads chunk g ^ (row & 7) of the same row).
-template <typename T, int WPT>
-__device__ __forceinline__ void copy_tile(const T *data, int64_t num_vecs, int V, int C, int64_t tl, int wib, int lane,
+// The copy of tile tl (rows tl*64 ...) into `buf` by one wave: the tile's
+// 16-byte chunks, each instruction 1 KB of consecutive bytes straight to LDS
+// (global_load_lds_dwordx4: no registers, tracked by vmcnt).  C = row bytes / 16;
+// swz: the placement above (then C % 8 == 0, and the lane of LDS chunk g loads
+// chunk g ^ (row & 7) of the same row).
+template <typename T>
+__device__ __forceinline__ void copy_tile(const T *data, int64_t num_vecs, int V, int C, int64_t tl, int lane,
                                           unsigned char *buf, bool swz)
 {
     const uint4 *src = reinterpret_cast<const uint4 *>(data + tl * kWave * (int64_t)V);
@@ -41,7 +41,7 @@ __device__ __forceinline__ void copy_tile(const T *data, int64_t num_vecs, int V
     // the last tile may be short: its missing rows re-read the last chunk
     const int64_t last = (rows_left < kWave ? rows_left : kWave) * C - 1;
     const float rc = 1.0f / (float)C;
-    for (int k = wib; k < C; k += WPT) {
+    for (int k = 0; k < C; ++k) {
         int g = k * kWave + lane;
         if (swz) g ^= (int)(((float)g + 0.5f) * rc) & 7; // row g / C (exact: g < 2048, C <= 32)
         __builtin_amdgcn_global_load_lds(static_cast<const void *>(src + (g < last ? g : last)),
@@ -63,40 +63,28 @@ __device__ __forceinline__ T chunk_elem(const uint4 &v, int e)
 
 // lost + (d & m != 0 ? popc(m) : 0) as AND, (AND-OR), MIN, MAD_U24 with the
 // mask and its popcount in SGPRs (one scalar operand per instruction).
-// ORDERED keeps the steps in program order with the other volatile asm of the
+// Volatile: the steps stay in program order with the other volatile asm of the
 // loop, so the scalar loads of the next column stay ahead of them and their
 // wait behind them.
-#define IBP_LOST_STEP64                                                                                                \
-    "v_and_b32 %0, %2, %3\n\t"                                                                                          \
-    "v_and_or_b32 %0, %4, %5, %0\n\t"                                                                                   \
-    "v_min_u32 %0, 1, %0\n\t"                                                                                           \
-    "v_mad_u32_u24 %1, %0, %6, %1"
-#define IBP_LOST_STEP32                                                                                                \
-    "v_and_b32 %0, %2, %3\n\t"                                                                                          \
-    "v_min_u32 %0, 1, %0\n\t"                                                                                           \
-    "v_mad_u32_u24 %1, %0, %4, %1"
-template <bool ORDERED = false>
 __device__ __forceinline__ uint32_t lost_step(uint64_t d, uint64_t m, uint32_t pc, uint32_t lost)
 {
     uint32_t z;
-    if constexpr (ORDERED)
-        asm volatile(IBP_LOST_STEP64
-                     : "=&v"(z), "+v"(lost)
-                     : "s"((uint32_t)m), "v"((uint32_t)d), "v"((uint32_t)(d >> 32)), "s"((uint32_t)(m >> 32)), "s"(pc));
-    else
-        asm(IBP_LOST_STEP64
-            : "=&v"(z), "+v"(lost)
-            : "s"((uint32_t)m), "v"((uint32_t)d), "v"((uint32_t)(d >> 32)), "s"((uint32_t)(m >> 32)), "s"(pc));
+    asm volatile("v_and_b32 %0, %2, %3\n\t"
+                 "v_and_or_b32 %0, %4, %5, %0\n\t"
+                 "v_min_u32 %0, 1, %0\n\t"
+                 "v_mad_u32_u24 %1, %0, %6, %1"
+                 : "=&v"(z), "+v"(lost)
+                 : "s"((uint32_t)m), "v"((uint32_t)d), "v"((uint32_t)(d >> 32)), "s"((uint32_t)(m >> 32)), "s"(pc));
     return lost;
 }
-template <bool ORDERED = false>
 __device__ __forceinline__ uint32_t lost_step(uint32_t d, uint32_t m, uint32_t pc, uint32_t lost)
 {
     uint32_t z;
-    if constexpr (ORDERED)
-        asm volatile(IBP_LOST_STEP32 : "=&v"(z), "+v"(lost) : "s"(m), "v"(d), "s"(pc));
-    else
-        asm(IBP_LOST_STEP32 : "=&v"(z), "+v"(lost) : "s"(m), "v"(d), "s"(pc));
+    asm volatile("v_and_b32 %0, %2, %3\n\t"
+                 "v_min_u32 %0, 1, %0\n\t"
+                 "v_mad_u32_u24 %1, %0, %4, %1"
+                 : "=&v"(z), "+v"(lost)
+                 : "s"(m), "v"(d), "s"(pc));
     return lost;
 }
 
