@@ -11,6 +11,7 @@
  * same slot format with 8- and 16-bit words.
  * Index arrays hold `index_bytes` = 4 (int32) or 8 (int64) signed entries.
  * Data pointers may be device memory or pinned (hipHostMalloc) host memory.
+ * What a call reads must not change until its work is done.
  *
  * Each declaration names the reference interface it replaces
  * (AKKamath/InvariantBitPacking, file:line).
@@ -188,7 +189,7 @@ int ibp_compress_ex(int elem_bytes, const void *input, void *output, int64_t num
  * default to half a block per CU: enough to saturate PCIe, leaving CUs to other
  * streams' kernels.  Out-of-range indices produce zero rows and are counted
  * (ibp_index_errors).  No allocation, no host synchronisation: safe under
- * stream capture.  What the call reads must not change until its work is done. */
+ * stream capture. */
 int ibp_decompress_fetch(int elem_bytes, void *out, const void *comp, int64_t num_vecs,
                          int64_t vec_size, const void *mask, const void *bitval,
                          const int32_t *bitmask, const void *index, int index_bytes, int64_t n,

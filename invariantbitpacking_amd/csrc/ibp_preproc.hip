@@ -565,7 +565,7 @@ __global__ __launch_bounds__(SPLIT == 1 ? 256 : 64 * SPLIT) void score_slices_ke
 }
 
 // Launch for nt thresholds (1, or the sweep), N > 0.  Four waves per SIMD fit
-// (100 registers); a fifth gave nothing.
+// (the sweep takes 84 to 128 registers, by the slice); a fifth gave nothing.
 template <typename T>
 void launch_score_slices(const T *data, int64_t N, int64_t V, const uint32_t *recs, int nt, Sums *sums, const T *masks,
                          const T *bitvals, T *mask, T *bitval, int32_t *chosen, int num_cus, hipStream_t stream)

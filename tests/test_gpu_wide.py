@@ -107,6 +107,7 @@ def test_wide_clusters_inside_a_batch(ibp, oracle, w, v, k):
 
 
 # team sizes (1, 2, 4, 8 waves) follow from the chunks and the rows; 32 KiB is the widest row a team packs
+# (here rows of 512 columns to 32 KiB go to teams, of eight waves; test_gpu_pack_teams.py has the other teams)
 @pytest.mark.parametrize("w,v", [(4, 65), (4, 129), (4, 255), (4, 513), (4, 2049), (4, 8192), (4, 8193),
                                  (8, 65), (8, 127), (8, 256), (8, 257), (8, 1030), (8, 4096), (8, 4097)])
 @pytest.mark.parametrize("n", [37, 4500])
