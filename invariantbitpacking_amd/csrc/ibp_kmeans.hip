@@ -798,9 +798,9 @@ KmPlan plan_kmeans(const DeviceInfo &dev, int w, int64_t N, int64_t V, int K, bo
     // (ibp_kmeans_mfma.h).  Waves per 16-row tile: more while the tiles alone
     // leave the chip short of waves and each wave keeps two steps of 64 bytes;
     // 16 for rows of 2 MiB and more, whose sums would leave the exact range of
-    // one accumulator.  (A launch is below 2^32 threads, and the tiles take four
-    // per row at least.)
-    pl.mfma = K <= kMfmaK && N > 0 && N < (int64_t)1 << 30;
+    // one accumulator.  (A launch is below 2^32 threads, and the tiles take 512
+    // per 128 rows at least.)
+    pl.mfma = K <= kMfmaK && N > 0 && (N + 127) / 128 * 512 < (int64_t)1 << 32;
     const int64_t tiles16 = (N + 15) / 16;
     pl.col_tiles = (VD + 15) / 16;
     pl.row_blocks = (N + 127) / 128;

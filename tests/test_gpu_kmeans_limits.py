@@ -13,12 +13,13 @@ def ibp():
     return m
 
 
-def test_rows_beyond_one_launch_of_tiles(ibp):
+# 512 threads per 128 rows, begun ones too: 2^32 - 512 are the most that a launch of tiles takes
+@pytest.mark.parametrize("n", [(1 << 30) - 128, (1 << 30) - 127, (1 << 30) + 5])
+def test_rows_beyond_one_launch_of_tiles(ibp, n):
     """2^30 rows of one column: four threads a row would be 2^32, more than a launch takes."""
-    n = (1 << 30) + 5
     values = torch.tensor([0x0000ffff, 0x0000fff0, 0x7fff0000], dtype=torch.int32, device="cuda")
     x = values[(torch.arange(n, dtype=torch.int32, device="cuda") % 7 % 3).long()].view(n, 1)
-    print("2^30 rows", flush=True)
+    print("rows", n, flush=True)
     mask, bitval, cl = ibp.preprocess_kmeans(x, 2, seed=3)
     cl = cl.cuda()
     of = [cl[k::7] for k in range(7)]  # row i holds values[i % 7 % 3]
