@@ -25,8 +25,8 @@
 // mask rows 92 -> 47 us, 27,000 rows of 99 words with scattered masks 32.6 -> 21.5 us.
 //
 // With a mask row per cluster the team looks through a window of rows and
-// batches those of one mask row (raw rows need none) where they are most of it;
-// the others go to a wave per row, or to two.
+// batches those of one mask row (raw rows need none) where such rows are most of
+// the call's; the others go to a wave per row, or to two.
 #pragma once
 
 #include "ibp_fetch_dev.h"
@@ -605,15 +605,20 @@ struct WideWindow {
     uint64_t ok; // the rows that are not refused
     int nrows;
 
+    // i: this lane's output row (places past the last one: any row).
     template <typename IdxT, int LAYOUT>
-    __device__ __forceinline__ void load(const FetchParams &p, int64_t b, int64_t e)
+    __device__ __forceinline__ void load(const FetchParams &p, int64_t i, int rows)
     {
-        nrows = (int)(e - b);
-        const int r = lane_id() < nrows ? lane_id() : 0;
-        const int64_t s = load_index<IdxT>(p.index, b + r);
+        nrows = rows;
+        const int64_t s = load_index<IdxT>(p.index, i);
         m = decode_meta<T, LAYOUT>(p, s, true, load_meta<LAYOUT>(p, s, true));
         key = !m.ok ? -2 : m.packed ? m.cl : -1;
         count();
+    }
+    template <typename IdxT, int LAYOUT>
+    __device__ __forceinline__ void load_window(const FetchParams &p, int64_t b, int64_t e)
+    {
+        load<IdxT, LAYOUT>(p, b + (lane_id() < (int)(e - b) ? lane_id() : 0), (int)(e - b));
     }
     __device__ __forceinline__ void count()
     {
@@ -632,27 +637,63 @@ struct WideWindow {
     }
     // The rows that one batch may hold beside row r, which is not refused.
     __device__ __forceinline__ uint64_t alike(int r) const { return ballot(key == readlane(key, r)) & ok; }
-    // The rows that a team takes: those of one mask row and the raw ones, if
-    // they are `least` at least; else none.
-    __device__ __forceinline__ uint64_t batched(int least) const
+    // The raw rows and those of mask rows with `each` rows or more, or with all
+    // but a quarter of the window's together with the raw ones.
+    __device__ __forceinline__ uint64_t alike_rows(int each) const
     {
         const uint64_t raw = ballot(key == -1) & ok;
-        uint64_t left = ok & ~raw;
+        uint64_t take = raw, left = ok & ~raw;
         const int nraw = __builtin_popcountll(raw);
-        while (__builtin_popcountll(left) + nraw >= least) { // uniform
-            if (!left) return raw;
+        while (__builtin_popcountll(left) >= each || __builtin_popcountll(left | raw) * 4 >= nrows * 3) { // uniform
+            if (!left) break;
             const uint64_t same = alike(__builtin_ctzll(left));
-            if (__builtin_popcountll(same) + nraw >= least) return same | raw;
+            const int n = __builtin_popcountll(same);
             left &= ~same;
+            if (n >= each || (n + nraw) * 4 >= nrows * 3) take |= same;
         }
-        return 0;
+        return take;
     }
-    __device__ __forceinline__ uint64_t batched() const { return batched((3 * nrows + 3) / 4); }
+    // Whether all rows go together: one mask row, and raw ones.  (Without a
+    // branch, which takes a register more.)
+    __device__ __forceinline__ bool uniform() const
+    {
+        const uint64_t packed = ballot(key >= 0) & ok;
+        return __builtin_popcountll(ok) >= nrows &&
+               (packed == 0 || alike(__builtin_ctzll(packed | 1ull << 63)) == packed);
+    }
 };
+
+// Whether windows of `rows` rows (more than kWideRows) go to teams at all, from
+// 64 rows of the call (four stretches of 16): mask rows that a window is to hold
+// twelve rows of have to make three quarters of them; of windows of 16, one
+// mask row nearly all of them.  Every wave that asks finds the same answer.
+// (By each window for itself, chance gives the teams a few windows of tables
+// whose rows should all go to a wave each, which then wait for them: 8192 rows of
+// 800 doubles of two mask rows 62 us, a wave per row 40, now 45.)
+template <typename T, typename IdxT, int LAYOUT>
+__device__ __forceinline__ bool windows_pay(const FetchParams &p, int rows)
+{
+    WideWindow<T> sample;
+    const int64_t i = lane_id() / 16 * (p.n / 4) + lane_id() % 16;
+    sample.template load<IdxT, LAYOUT>(p, i < p.n ? i : p.n - 1, kWave);
+    const uint64_t raw = ballot(sample.key == -1);
+    const int each = rows <= 16 ? 60 : kWave * 12 / rows, least = rows <= 16 ? 60 : 48;
+    uint64_t left = sample.ok & ~raw;
+    const int nraw = __builtin_popcountll(raw);
+    int take = nraw;
+    while (left && take + __builtin_popcountll(left) >= least) { // uniform
+        const uint64_t same = sample.alike(__builtin_ctzll(left));
+        const int n = __builtin_popcountll(same);
+        left &= ~same;
+        if (n >= each || n + nraw >= least) take += n;
+    }
+    return take >= least;
+}
 
 // A window's rows in the team's LDS: where the stored rows start, their bytes,
 // their keys.
 constexpr int kWindowLdsWords = 5 * kWideWindow;
+constexpr int kWindowAlike = 6; // rows of one mask row that a team takes from a window, at least
 
 // The part of a window that a team of two waves or more takes, in batches of
 // rows alike.  WHOLE (windows of kWideRows at most): all of it, in batches if all
@@ -675,7 +716,7 @@ __device__ __forceinline__ void fetch_wide_window(const FetchParams &p, int64_t 
     WideWindow<T> win;
     batch.sync(); // the window before this one is done
     if (slot == 0) {
-        win.template load<IdxT, LAYOUT>(p, b, e);
+        win.template load_window<IdxT, LAYOUT>(p, b, e);
         start[lane_id()] = win.m.word * (int64_t)sizeof(T);
         stored[lane_id()] = win.m.len * (int64_t)sizeof(T);
         keys[lane_id()] = win.key;
@@ -685,7 +726,7 @@ __device__ __forceinline__ void fetch_wide_window(const FetchParams &p, int64_t 
     win.key = keys[lane_id()];
     win.count();
     if constexpr (WHOLE) {
-        if (!win.batched(win.nrows)) {
+        if (!win.uniform()) {
             // Two waves a row.
             const WideBatch<T, LAYOUT, NT, 1, true> one(p, 2, slot & 1, lds + (slot >> 1) * kWideStride);
             for (int r0 = 0; r0 < win.nrows; r0 += team / 2) {
@@ -705,7 +746,7 @@ __device__ __forceinline__ void fetch_wide_window(const FetchParams &p, int64_t 
             return;
         }
     }
-    for (uint64_t left = WHOLE ? win.ok : win.batched(); left;) {
+    for (uint64_t left = WHOLE ? win.ok : win.alike_rows(kWindowAlike); left;) {
         const int head = __builtin_ctzll(left);
         uint64_t alike = win.alike(head) & left;
         left &= ~alike;

@@ -10,6 +10,19 @@ namespace ibp {
 // a window that shares a mask row (fetch_wide_rest_kernel takes the others).
 enum : int { kBatches, kWholeWindows, kWindowParts };
 
+// windows_pay by one wave for the block.
+template <typename T, typename IdxT, int LAYOUT>
+__device__ __forceinline__ bool block_windows_pay(const FetchParams &p, int rows)
+{
+    __shared__ int pay;
+    if (wave_in_block_id() == 0) {
+        const bool yes = windows_pay<T, IdxT, LAYOUT>(p, rows);
+        if (lane_id() == 0) pay = yes;
+    }
+    __syncthreads();
+    return readfirstlane((int64_t)pay) != 0;
+}
+
 // Batches (windows) of rows_per_batch rows.  team > 1: a block is one team;
 // team = 1 (not with windows): each of a block's waves takes its own batches.
 template <typename T, typename IdxT, int LAYOUT, bool NT, int TAKE>
@@ -18,6 +31,9 @@ __global__ __launch_bounds__(64 * kWideMaxTeam, 4) void fetch_wide_kernel(FetchP
     __shared__ uint32_t lds[kWideSolo][kWideLdsWords];
     __shared__ __align__(8) uint32_t window[TAKE == kBatches ? 1 : kWindowLdsWords];
     const int wib = wave_in_block_id();
+    if constexpr (TAKE == kWindowParts) {
+        if (!block_windows_pay<T, IdxT, LAYOUT>(p, rows_per_batch)) return;
+    }
     const int64_t first = team > 1 ? (int64_t)blockIdx.x : global_wave_id();
     const int64_t step = team > 1 ? (int64_t)gridDim.x : (int64_t)gridDim.x * (blockDim.x / kWave);
     for (int64_t b = first * rows_per_batch; b < p.n; b += step * rows_per_batch) {
@@ -30,19 +46,25 @@ __global__ __launch_bounds__(64 * kWideMaxTeam, 4) void fetch_wide_kernel(FetchP
 }
 
 // A wave per row for the rows of windows of `rows` rows (a power of two) that
-// the teams leave.  (In the teams' kernel they had half the waves in flight, and
-// their code cost it scratch memory: 8192 rows of 800 doubles with 16 evenly used
-// mask rows 56 us, so 45; a wave per row for all of them 40.)
+// the teams leave, which is all of them where windows do not pay.  (In the
+// teams' kernel they had half the waves in flight, and their code cost it
+// scratch memory: 8192 rows of 800 doubles of 16 evenly used mask rows 56 us, so
+// 43, to which the launch that finds nothing to do adds 3; a wave per row 40.)
 template <typename T, typename IdxT, int LAYOUT>
 __global__ __launch_bounds__(256) void fetch_wide_rest_kernel(FetchParams p, int rows)
 {
+    const bool teams = block_windows_pay<T, IdxT, LAYOUT>(p, rows);
     const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / kWave);
+    if (!teams) {
+        fetch_large_range<T, IdxT, LAYOUT>(p, global_wave_id(), p.n, nwaves);
+        return;
+    }
     for (int64_t i = global_wave_id(); i < p.n; i += nwaves) {
         const int64_t b = i & ~(int64_t)(rows - 1);
         const int r = (int)(i - b);
         WideWindow<T> win;
-        win.template load<IdxT, LAYOUT>(p, b, b + rows < p.n ? b + rows : p.n);
-        if ((win.batched() >> r) & 1) continue; // uniform
+        win.template load_window<IdxT, LAYOUT>(p, b, b + rows < p.n ? b + rows : p.n);
+        if ((win.alike_rows(kWindowAlike) >> r) & 1) continue; // uniform
         fetch_large_row<T>(p, i, win.row(r));
     }
 }
@@ -100,7 +122,8 @@ void launch_layout(const FetchParams &p, int layout, const WideShape &w, int nbl
 // rows of one mask row (weights, node features, embeddings mostly): 2000, 4096
 // and 30,000 rows of 800 doubles 16, 23 and 130 us by a wave per row and 13, 15
 // and 87 by teams, of 2752 doubles (16,000) 51, 75 and 240 and 24, 33 and 135.
-// Sixteen evenly used: 16, 24, 130 and 15, 25, 140; 52, 76, 239 and 38, 76, 244.
+// Sixteen evenly used: 16, 24, 130 and 15, 25, 140; 52, 76, 239 and 38, 76, 241;
+// two (12,000 rows) 58 and 54, 181 and 112.
 // (With blocks of one wave, by nthreads, a window has no team.)
 bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes, int nthreads)
 {

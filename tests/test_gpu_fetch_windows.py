@@ -70,3 +70,30 @@ def test_rows_by_cluster_use(ibp, oracle, usage, w, v, n):
         got = ibp.decompress(torch.from_numpy(stream).cuda(), torch.from_numpy(off).cuda(), m, b, dev, v, ix, clusters=c)
         assert np.array_equal(got.cpu().numpy().reshape(want.shape), want), "stream"
         assert ibp.index_errors(reset=True) == wrong
+
+
+# windows of 16, 32 and 64 rows; whether they go to teams is read from four stretches of 16 rows
+@pytest.mark.parametrize("n", [4200, 9001, 20003])
+@pytest.mark.parametrize("order", ["sampled alike", "sampled mixed", "sorted", "refused"])
+def test_rows_unlike_the_sample(ibp, oracle, n, order):
+    rng = np.random.default_rng(n + len(order))
+    x, mask, bitval, cl = table(8, 800, 5, "even", rng)
+    comp, bm = oracle.compress(x.view("i8"), mask.view("i8"), bitval.view("i8"), clusters=cl)
+    idx = rng.integers(0, ROWS, size=n)
+    packed = np.unpackbits(bm.view(np.uint8), bitorder="little")[:ROWS] == 1
+    of = [np.flatnonzero((cl == c) & packed) for c in range(5)]
+    sample = (np.arange(64) // 16 * (n // 4) + np.arange(64) % 16)
+    if order == "sampled alike":
+        idx[sample] = rng.choice(of[0], size=64)
+    elif order == "sampled mixed":
+        idx = rng.choice(of[1], size=n)
+        idx[sample] = rng.integers(0, ROWS, size=64)
+    elif order == "sorted":
+        idx = idx[np.argsort(cl[idx], kind="stable")]
+    else:
+        idx[sample] = -1
+    args = [torch.from_numpy(a).cuda() for a in (comp.view("i8"), mask.view("i8"), bitval.view("i8"), bm.view(np.int32))]
+    print("unlike the sample", n, order, flush=True)
+    got = ibp.decompress_fetch(*args, torch.device("cuda"), None, torch.from_numpy(idx).cuda(),
+                               clusters=torch.from_numpy(cl).cuda())
+    assert np.array_equal(got.cpu().numpy(), expect(x.view("i8"), idx))
