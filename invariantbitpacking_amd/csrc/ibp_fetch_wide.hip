@@ -125,11 +125,17 @@ void launch_layout(const FetchParams &p, int layout, const WideShape &w, int nbl
 // Sixteen evenly used: 16, 24, 130 and 15, 25, 140; 52, 76, 239 and 38, 76, 241;
 // two (12,000 rows) 58 and 54, 181 and 112.
 // (With blocks of one wave, by nthreads, a window has no team.)
+// Over PCIe rows of up to three chunks of 64-bit words stay with a wave per row,
+// whose reads of a row come from one wave in address order (20,000 and 60,000
+// embeddings of 66 doubles in a stream 145 and 385 us, by teams 159 and 404, of
+// 100 188 and 508, 195 and 532; of 129 221 and 594, 229 and 630; of 160 it turns:
+// 259 and 709, 245 and 672).  Of 32-bit words teams are as fast or faster.
 bool fetch_wide_pays(const FetchParams &p, int layout, int elem_bytes, int nthreads)
 {
     if (p.vec_size <= kWave || elem_bytes < 4) return false;
     const int64_t row_bytes = p.vec_size * elem_bytes;
     if (layout & kLayoutClustered) return row_bytes >= 6144 && (nthreads <= 0 || nthreads >= 2 * kWave);
+    if (p.host_rows && elem_bytes == 8 && p.vec_size < 160) return false;
     return p.vec_size >= 512 || p.n >= ((int64_t)8 << 20) / row_bytes;
 }
 
