@@ -535,10 +535,10 @@ __device__ __forceinline__ void fetch_small_range_meta(const FetchParams &p, con
     }
 }
 
-// Fetches and unpacks output row i (its stored row's place and kind in me) of a
-// table with rows of any length, one 64-element chunk at a time.  Wave-uniform.
-template <typename T>
-__device__ __forceinline__ void fetch_large_row(const FetchParams &p, int64_t i, const RowMeta &me)
+// Fetches and unpacks output row i (its stored row's place and kind by meta()) of
+// a table with rows of any length, one 64-element chunk at a time.  Wave-uniform.
+template <typename T, typename Meta>
+__device__ __forceinline__ void fetch_large_row(const FetchParams &p, int64_t i, Meta meta)
 {
     constexpr int B = Bits<T>::B;
     constexpr int FLAGS_PER_WORD = B;
@@ -547,6 +547,7 @@ __device__ __forceinline__ void fetch_large_row(const FetchParams &p, int64_t i,
     const int64_t Hw = header_bytes(V, (int)sizeof(T)) / (int64_t)sizeof(T);
     T *dst = (T *)p.out + i * V;
 
+    const RowMeta me = meta();
     if (!me.ok) {
         for (int64_t k = lane; k < V; k += kWave) dst[k] = T(0);
         if (p.err && lane == 0) atomicAdd(p.err, 1ull);
@@ -634,7 +635,7 @@ __device__ __forceinline__ void fetch_large_range(const FetchParams &p, int64_t 
     int64_t s = readfirstlane(load_index<IdxT>(p.index, b));
     for (int64_t i = b; i < e; i += step) {
         const int64_t nxt = i + step < e ? readfirstlane(load_index<IdxT>(p.index, i + step)) : 0;
-        fetch_large_row<T>(p, i, decode_meta<T, LAYOUT>(p, s, true, load_meta<LAYOUT>(p, s, true)));
+        fetch_large_row<T>(p, i, [&] { return decode_meta<T, LAYOUT>(p, s, true, load_meta<LAYOUT>(p, s, true)); });
         s = nxt;
     }
 }

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void fetch_wide_rest_kernel(FetchParams p, int
         WideWindow<T> win;
         win.template load_window<IdxT, LAYOUT>(p, b, b + rows < p.n ? b + rows : p.n);
         if ((win.alike_rows(kWindowAlike) >> r) & 1) continue; // uniform
-        fetch_large_row<T>(p, i, win.row(r));
+        fetch_large_row<T>(p, i, [&] { return win.row(r); });
     }
 }
 
